@@ -10,6 +10,8 @@
 //                  extend each other): scores, chunk max, exp, chunk sum and
 //                  chunk-weighted V of each row; passes of at most 8 rows
 //                  also quantize and store their own K/V rows here
+//   k_attn_tile    the same per (head, chunk, 32 rows) on the fp32 matrix
+//                  core, for prompt passes before anything leaves the window
 //   k_attn_chunk   the same per (row, head, chunk), for batched passes of
 //                  more than 8 rows
 //   k_attn_seq     the same per (head, chunk, group of a sequence's rows)
@@ -1343,6 +1345,293 @@ __global__ __launch_bounds__(512) void k_attn_group(const PassDesc* __restrict__
     attn_group_body<PARTS, FUSED, NR, false>(pd, g, kv, layer, M, q, kself, vself, S, s_stride, Up, cstride, pf,
                                              LLIn{}, blockIdx.x, blockIdx.y, blockIdx.x + blockIdx.y * gridDim.x,
                                              gridDim.x, smem);
+}
+
+// ------------------------------------------------- row-tile attention
+
+typedef float pf_v16f __attribute__((ext_vector_type(16)));
+typedef float pf_v32f __attribute__((ext_vector_type(32)));
+
+// LDS of k_attn_tile (bytes): the tile's queries [hd / 4][32] float4
+// (swizzled) and the chunk's V rows [256][hd], reused for the sub-chunks'
+// partial sums [4][32][64]; then the V scales [256], the rows' sub-chunk
+// maxima and sums [2][4][32] and self weights [32].
+__host__ __device__ constexpr uint32_t at_region(uint32_t hd) { return hd * 128u + 256u * hd > 32768u ? hd * 384u : 32768u; }
+__host__ __device__ constexpr uint32_t at_smem(uint32_t hd) { return at_region(hd) + (256u + 2u * 128u + 32u) * 4u; }
+
+// Engine attention (the first stage above) of a prompt pass whose rows'
+// lists are plain prefixes: every row sees the positions before its own and
+// nothing has left the window (row at position p: C = p entries, entry j at
+// position j).  One workgroup per (head, 256-entry chunk, 32 pass rows); wave
+// s takes sub-chunk s.
+//
+// Both products run on the matrix core with v_mfma_f32_32x32x1_2b_f32, whose
+// one step rounds as one fmaf per element (denormals and cancellations
+// included), so a chain of them is k_attn_group's fmaf chain bit for bit:
+//   scores  A = the sub-chunk's 64 converted keys (lane = entry), B = the
+//           32 rows' query element: one MFMA per query element, in order.
+//           The result has lane = row, so maxima, exp and the CANON(4) tree
+//           (offsets 32, 16, 8, 2, 1 between registers, 4 between the wave's
+//           halves) stay in registers.
+//   V       A = the 32 rows' weights of one entry (both halves), B = the
+//           entry's converted V row, 64 dims per MFMA, entries in order.
+// The self score and self V term are formed apart as in k_attn_group.
+//
+// What bounds it: fp32 issue.  An MFMA takes 64 cycles for 2048 FMAs (32.8 ns
+// measured), twice the VALU's rate without packed fp32, and fp32 MFMAs and
+// VALU instructions do not overlap (4 v_fma_f32 beside each MFMA: 32.8 -> 42.9
+// ns), so the two conversion steps per MFMA and the exps count in full: 256
+// MFMAs (8.4 us) and about 1500 VALU instructions (3.2 us) per wave at
+// head_dim 128.  In k_attn_group the VALU runs the chains and both conversions
+// for at most 4 rows per loaded chunk.  Three workgroups per CU (50 KB of LDS).
+// Measured per launch of 256 rows (16 heads of 128): 23.6 us at 2 chunks, 95
+// at 16, 134 at 23, 10 us per 256 workgroups once the chip is full; over a
+// 6000-token prompt 81 us on average, where k_attn_group took 490.
+template <int PARTS>
+__global__ __launch_bounds__(256, 3) void k_attn_tile(const PassDesc* __restrict__ pd, KvGeom g, KvPlanes kv,
+                                                      uint32_t layer, uint32_t M, uint32_t tiles, uint32_t n_groups,
+                                                      const float* __restrict__ q, const float* __restrict__ kself,
+                                                      const float* __restrict__ vself, float* __restrict__ S,
+                                                      uint32_t s_stride, float* __restrict__ Up, uint32_t cstride) {
+    constexpr uint32_t hd = 16 * PARTS, NT = hd / 64u, K4 = hd / 4u;
+    __shared__ __align__(16) uint8_t smem[at_smem(hd)];
+    float4* qt = reinterpret_cast<float4*>(smem);                       // [K4][32], row r at r ^ (k4 & 31)
+    uint8_t* vt = smem + hd * 128u;                                     // [256][hd]
+    float* xw = reinterpret_cast<float*>(smem);                         // [4][32][64], after the V chains
+    float* vsc = reinterpret_cast<float*>(smem + at_region(hd));        // [256]
+    float* mxs = vsc + 256;                                             // [4][32]
+    float* sms = mxs + 128;                                             // [4][32]
+    float* psf = sms + 128;                                             // [32]
+
+    // workgroup b runs on XCD b mod 8: a head's tiles and chunks share an L2
+    const uint32_t slot = blockIdx.x >> 3, grp = (slot / tiles) * 8u + (blockIdx.x & 7u), m0 = 32u * (slot % tiles);
+    if (grp >= n_groups) return;
+    const PassHead ph = pass_head(pd);
+    const uint32_t H = g.n_heads, h = grp % H, c = grp / H, j0 = 256u * c, D = H * hd;
+    const uint32_t nrow = min(32u, M - m0), p0 = ph.pos0 + m0, plast = p0 + nrow - 1u;
+    if (j0 > plast) return;                                             // past the last row's self entry
+    const uint32_t t = threadIdx.x, lane = t & 63u, r = lane & 31u, hh = lane >> 5;
+    const uint32_t sub = __builtin_amdgcn_readfirstlane(t >> 6), jb = j0 + 64u * sub;
+    const size_t prow = plane_index(g, ph.seq0, layer, h) * g.rows;
+    // plane row of entry j, clamped to the entries the last row sees
+    auto erow = [&](uint32_t j) -> size_t {
+        const uint32_t e = min(j, plast > 0u ? plast - 1u : 0u);
+        return prow + (e < g.sink_size ? e : e - g.sink_size + KV_SINK_ROWS);
+    };
+
+    // ---- loads: this lane's key, the sub-chunk's V rows, the queries
+    int4 kw[PARTS], vw[PARTS];
+    const size_t er = erow(jb + lane);
+#pragma unroll
+    for (int p = 0; p < PARTS; p++) kw[p] = reinterpret_cast<const int4*>(kv.k + er * hd)[p];
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)PARTS; i++) {
+        const uint32_t pi = lane + 64u * i;
+        vw[i] = reinterpret_cast<const int4*>(kv.v + erow(jb + pi / PARTS) * hd)[pi % PARTS];
+    }
+    const bool live = jb + lane < plast;                                // scales 0 past the entries
+    const float ks = live ? kv.ks[er] : 0.0f, vs = live ? kv.vs[er] : 0.0f;
+    float4 qv[K4 / 8u];
+#pragma unroll
+    for (uint32_t i = 0; i < K4 / 8u; i++) {
+        const uint32_t x = t + 256u * i, m = min(x / K4, nrow - 1u);
+        qv[i] = *reinterpret_cast<const float4*>(q + (size_t)(m0 + m) * D + h * hd + 4u * (x % K4));
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)PARTS; i++)
+        *reinterpret_cast<int4*>(vt + (size_t)64u * sub * hd + 16u * (lane + 64u * i)) = vw[i];
+    vsc[t] = vs;
+#pragma unroll
+    for (uint32_t i = 0; i < K4 / 8u; i++) {
+        const uint32_t x = t + 256u * i, k4 = x % K4;
+        qt[32u * k4 + ((x / K4) ^ (k4 & 31u))] = qv[i];
+    }
+    __syncthreads();
+
+    // ---- scores: register 16 b + i of lane (r, hh) is entry
+    // jb + 32 b + 8 (i / 4) + 4 hh + i % 4 of row r
+    const uint32_t p = p0 + r;                                          // row r's position (its list's self index)
+    const bool on = jb <= plast;                                        // the sub-chunk holds an entry of some row
+    const bool diag = jb + 63u >= p0;                                   // ... and may pass a row's list end
+    pf_v32f s = {};
+    float mx = -__builtin_inff();
+    if (on) {
+#pragma unroll
+        for (uint32_t k4 = 0; k4 < K4; k4++) {
+            const float4 q4 = qt[32u * k4 + (r ^ (k4 & 31u))];
+            const int4 w4 = kw[k4 >> 2];
+            const int w = (k4 & 3u) == 0u ? w4.x : ((k4 & 3u) == 1u ? w4.y : ((k4 & 3u) == 2u ? w4.z : w4.w));
+            const float qe[4] = {q4.x, q4.y, q4.z, q4.w};
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+                s = __builtin_amdgcn_mfma_f32_32x32x1f32((float)(int8_t)((w >> (8 * b)) & 0xFF) * ks, qe[b], s, 0, 0, 0);
+        }
+        const float scale = 1.0f / __builtin_sqrtf((float)hd);
+#pragma unroll
+        for (int i = 0; i < 32; i++) s[i] = s[i] * scale;
+        if (diag) {
+            float sd = 0.0f;
+            const float* kr = kself + (size_t)(m0 + min(r, nrow - 1u)) * D + h * hd;
+            const float4* qo = lds_opaque(qt);   // read again (kept from above they would spill)
+#pragma unroll
+            for (uint32_t kb = 0; kb < K4; kb += 8) {
+                float4 b[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++) b[u] = *reinterpret_cast<const float4*>(kr + 4u * (kb + u));
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++) {
+                    const float4 a = qo[32u * (kb + u) + (r ^ ((kb + u) & 31u))];
+                    sd = sd + a.x * b[u].x;
+                    sd = sd + a.y * b[u].y;
+                    sd = sd + a.z * b[u].z;
+                    sd = sd + a.w * b[u].w;
+                }
+            }
+            sd = sd * scale;
+#pragma unroll
+            for (uint32_t i = 0; i < 32; i++) {
+                const uint32_t j = jb + 32u * (i >> 4) + 8u * ((i >> 2) & 3u) + 4u * hh + (i & 3u);
+                s[i] = j < p ? s[i] : (j == p ? sd : -__builtin_inff());
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 32; i++) mx = fmaxf(mx, s[i]);
+        mx = fmaxf(mx, shfl_xor(mx, 32));
+    }
+    if (lane < 32u) mxs[sub * 32u + r] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(mxs[r], mxs[32u + r]), fmaxf(mxs[64u + r], mxs[96u + r]));
+
+    // ---- exp and the sub-chunk's sum (block_canon_sum's wave tree)
+    float tot = 0.0f;
+    if (on) {
+#pragma unroll
+        for (uint32_t i = 0; i < 32; i++) s[i] = expf_neg(s[i] - mx);
+        if (diag) {
+#pragma unroll
+            for (uint32_t i = 0; i < 32; i++) {
+                const uint32_t j = jb + 32u * (i >> 4) + 8u * ((i >> 2) & 3u) + 4u * hh + (i & 3u);
+                if (j > p) s[i] = 0.0f;
+            }
+        }
+        float a[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) a[i] = s[i] + s[16 + i];
+#pragma unroll
+        for (int i = 0; i < 8; i++) a[i] = a[i] + a[8 + i];
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i] = a[i] + a[4 + i];
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i] = a[i] + shfl_xor(a[i], 32);
+        tot = (a[0] + a[2]) + (a[1] + a[3]);
+        if (diag) {   // the self entry's weight leaves the V chain
+#pragma unroll
+            for (uint32_t i = 0; i < 32; i++) {
+                const uint32_t j = jb + 32u * (i >> 4) + 8u * ((i >> 2) & 3u) + 4u * hh + (i & 3u);
+                if (j == p) {
+                    psf[r] = s[i];
+                    s[i] = 0.0f;
+                }
+            }
+        }
+    }
+    if (lane < 32u) sms[sub * 32u + r] = tot;
+    __syncthreads();
+    if (t < nrow && j0 <= p0 + t) {
+        const size_t mh = (size_t)(m0 + t) * H + h;
+        S[mh * s_stride + 2u * c] = fmaxf(fmaxf(mxs[t], mxs[32u + t]), fmaxf(mxs[64u + t], mxs[96u + t]));
+        S[mh * s_stride + 2u * c + 1u] = (sms[t] + sms[64u + t]) + (sms[32u + t] + sms[96u + t]);
+    }
+
+    // ---- V chains: product n of lane l covers dim NT l + n; register
+    // 16 b + i of lane (x, hh) is row 8 (i / 4) + 4 hh + i % 4, dim
+    // NT (x + 32 b) + n
+    pf_v32f w[NT];
+#pragma unroll
+    for (uint32_t n = 0; n < NT; n++) w[n] = pf_v32f{};
+    if (on) {
+        const uint8_t* vl = lds_opaque(vt) + (size_t)64u * sub * hd + NT * lane;
+        const float* vc = lds_opaque(vsc) + 64u * sub;
+#pragma unroll
+        for (uint32_t o = 0; o < 64; o += 8) {   // entries o .. o + 7: registers i0 .. i0 + 3, both halves
+            const uint32_t i0 = 16u * (o >> 5) + 4u * ((o >> 3) & 3u);
+            float e[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) {
+                const auto pr = __builtin_amdgcn_permlane32_swap(f2u(s[i0 + u]), f2u(s[i0 + u]), false, false);
+                e[u] = u2f(pr[0]);
+                e[4 + u] = u2f(pr[1]);
+            }
+            const float4 c0 = *reinterpret_cast<const float4*>(vc + o), c1 = *reinterpret_cast<const float4*>(vc + o + 4u);
+            const float sc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+            uint32_t cd[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; u++)
+                cd[u] = NT == 2u ? *reinterpret_cast<const uint16_t*>(vl + (size_t)(o + u) * hd) : vl[(size_t)(o + u) * hd];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; u++)
+#pragma unroll
+                for (uint32_t n = 0; n < NT; n++)
+                    w[n] = __builtin_amdgcn_mfma_f32_32x32x1f32(e[u], (n ? cvt_i8_1(cd[u]) : cvt_i8_0(cd[u])) * sc[u], w[n], 0,
+                                                                0, 0);
+        }
+        if (diag) {
+            // the rows whose self entry is here add their own value's term;
+            // eight rows' loads are issued before any is used
+#pragma unroll
+            for (uint32_t ib = 0; ib < 32; ib += 8) {
+                float vr[8][NT], ps[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++) {
+                    const uint32_t i = ib + u, row = min(8u * ((i >> 2) & 3u) + 4u * hh + (i & 3u), nrow - 1u);
+                    const float* a = vself + (size_t)(m0 + row) * D + h * hd + NT * (r + 32u * (i >> 4));
+#pragma unroll
+                    for (uint32_t n = 0; n < NT; n++) vr[u][n] = a[n];
+                    ps[u] = psf[row];
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++) {
+                    const uint32_t i = ib + u, row = 8u * ((i >> 2) & 3u) + 4u * hh + (i & 3u);
+                    const bool mine = row < nrow && p0 + row - jb < 64u;
+#pragma unroll
+                    for (uint32_t n = 0; n < NT; n++)
+                        w[n][i] = mine ? __builtin_fmaf(ps[u], vr[u][n], w[n][i]) : w[n][i];
+                }
+            }
+        }
+    }
+    // ---- the sub-chunks' sums added in order, 64 dims at a time
+#pragma unroll
+    for (uint32_t b = 0; b < NT; b++) {
+        __syncthreads();                                                // the region's earlier contents are read
+#pragma unroll
+        for (uint32_t i = 0; i < 16; i++) {
+            const uint32_t row = 8u * (i >> 2) + 4u * hh + (i & 3u);
+            float* x = xw + (size_t)(sub * 32u + row) * 64u;
+            if constexpr (NT == 2u) {
+                *reinterpret_cast<float2*>(x + 2u * r) = make_float2(w[0][16u * b + i], w[1][16u * b + i]);
+            } else {
+                x[r] = w[0][i];
+                x[32u + r] = w[0][16u + i];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t i = 0; i < 2; i++) {
+            const uint32_t x = t + 256u * i, row = x >> 4, d4 = 4u * (x & 15u);
+            float4 u = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+            for (uint32_t y = 0; y < 4; y++) {
+                const float4 a = *reinterpret_cast<const float4*>(xw + (size_t)(y * 32u + row) * 64u + d4);
+                u.x = u.x + a.x;
+                u.y = u.y + a.y;
+                u.z = u.z + a.z;
+                u.w = u.w + a.w;
+            }
+            if (row < nrow && j0 <= p0 + row)
+                *reinterpret_cast<float4*>(Up + (((size_t)(m0 + row) * H + h) * cstride + c) * hd + 64u * b + d4) = u;
+        }
+    }
 }
 
 // Engine attention, second stage: the chunks of (row m, head h) merged left

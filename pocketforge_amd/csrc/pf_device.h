@@ -40,6 +40,38 @@ __device__ __forceinline__ float expf_c(float x) {
     return p * u2f((uint32_t)(k + 127) << 23);
 }
 
+// expf_c(x) for x <= 0 (or NaN) without its early returns: the same steps
+// for every x, then one select, for loops over many elements in registers (a
+// branch per element costs more than the unused steps).  ldexp is the
+// exponent-field product of expf_c: p * 2^k is a normal number for x >= -86.
+__device__ __forceinline__ float expf_neg(float x) {
+    const float kf = __builtin_rintf(x * 1.44269502162933349609375f);
+    float r = __builtin_fmaf(kf, -0.693145751953125f, x);
+    r = __builtin_fmaf(kf, -1.42860676533018704503775e-06f, r);
+    float p = 1.98412698412698412698e-4f;
+    p = __builtin_fmaf(p, r, 1.38888888888888888889e-3f);
+    p = __builtin_fmaf(p, r, 8.33333333333333333333e-3f);
+    p = __builtin_fmaf(p, r, 4.16666666666666666667e-2f);
+    p = __builtin_fmaf(p, r, 1.66666666666666666667e-1f);
+    p = __builtin_fmaf(p, r, 0.5f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    const float y = __builtin_amdgcn_ldexpf(p, (int)fmaxf(kf, -1024.0f));
+    return x < -86.0f ? 0.0f : y;
+}
+
+// Signed bytes 0 and 1 of a word as floats, one instruction each.
+__device__ __forceinline__ float cvt_i8_0(uint32_t w) {
+    float f;
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(f) : "v"(w));
+    return f;
+}
+__device__ __forceinline__ float cvt_i8_1(uint32_t w) {
+    float f;
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(f) : "v"(w));
+    return f;
+}
+
 // IEEE binary16 bits -> float: v_cvt_f32_f16, exact for every finite value
 // (subnormal halves included: this code is built without denormal flushing).
 __device__ __forceinline__ float h2f(uint16_t h) {

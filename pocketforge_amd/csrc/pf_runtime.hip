@@ -593,7 +593,24 @@ static bool attn_fused(uint32_t M) { return M <= AG_MAX_ROWS; }
 static void launch_attn(hipStream_t st, uint32_t hd, uint32_t M, uint32_t tasks, const PassDesc* pd,
                         const KvGeom& g, const KvPlanes& kv, uint32_t l, const float* q, const float* k,
                         const float* v, float* S, uint32_t s_stride, float* Wp, uint32_t cstride, Prefetch pf,
-                        bool batch, uint32_t gsize, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr) {
+                        bool batch, uint32_t gsize, bool prefix, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr) {
+    // k_attn_tile's time is one workgroup's (22 us at head_dim 128, 15 at 64)
+    // up to 256 workgroups, then 10 us per 256 more; k_attn_group's grows with
+    // its blocks of 4 rows: 11.5 / 21 / 29 / 114 us at 192 / 384 / 576 / 2560 of
+    // them (head_dim 128), 9 / 16 us at 16 / 192 (head_dim 64)
+    if (prefix && M > AG_MAX_ROWS && (M + 3) / 4 * tasks > (hd == 64 ? 192u : 384u)) {
+        // blocks b with equal b mod 8 (one XCD) hold whole (head, chunk)
+        // groups of 32-row tiles
+        const uint32_t tiles = (M + 31) / 32;
+        const dim3 grid(8 * tiles * ((tasks + 7) / 8));
+        if (hd == 64)
+            hipExtLaunchKernelGGL((k_attn_tile<4>), grid, dim3(256), 0, st, ev0, ev1, 0, pd, g, kv, l, M, tiles, tasks,
+                                  q, k, v, S, s_stride, Wp, cstride);
+        else
+            hipExtLaunchKernelGGL((k_attn_tile<8>), grid, dim3(256), 0, st, ev0, ev1, 0, pd, g, kv, l, M, tiles, tasks,
+                                  q, k, v, S, s_stride, Wp, cstride);
+        return;
+    }
     if (batch && M > AG_MAX_ROWS && gsize >= 2 && gsize <= AS_NR) {
         // groups of gsize consecutive positions of one sequence (a batched
         // verify pass): one block per (head, chunk, group) loads the union
@@ -2041,6 +2058,11 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
     const uint32_t ks = e->kmax;
     const bool tall = M > GEMV_MAX_M;
     const bool merge_in_o = M == 1 && D <= 2048;
+    // every row's list is a prefix of the last row's and holds one entry per
+    // earlier position: one sequence, every sink position stored, nothing past
+    // max_context, and the last row's window not yet full
+    const bool prefix = !batch && !e->capturing && g.sink_size <= KV_SINK_ROWS && pos_last <= g.max_context &&
+                        pos_last <= g.sink_size + g.window;
     // activation scales [4][rows] of the tall passes' row kernels
     float* as0 = e->as;                   // attention-norm act
     float* as1 = e->as + e->rows;         // attention output act
@@ -2252,7 +2274,7 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
             else qkv_attn_rows<8>(st, a, b, attn_tasks, aev0, aev1);
         } else {
             launch_attn(st, hd, M, attn_tasks, pd, g, e->kv, l, e->q, e->k, e->v, e->S, e->s_stride, e->Wp,
-                        e->cstride, opf, batch, batch ? e->batch_group : 0u, aev0, aev1);
+                        e->cstride, opf, batch, batch ? e->batch_group : 0u, prefix, aev0, aev1);
         }
         if (!merge_in_o && !tail)
             PF_PER1024_SWITCH(D, hipLaunchKernelGGL(k_attn_merge_quant<PER>, dim3(M + e->pf_blocks), dim3(1024), 0, st,

@@ -1,0 +1,47 @@
+"""Attention of prompt passes (more than 8 rows of one sequence): the cache
+and the next forward after one tall pass equal those after passes of at most
+8 rows, which run the other attention kernels (pinned to the oracle), bit for
+bit.  Heights and starts around the 32-row tile, the 64-entry sub-chunk and
+the 256-entry chunk, passes that end at the last position before the window
+is full and one past it, and sink sizes the prefix rule accepts and not."""
+import numpy as np
+import pytest
+
+import pocketforge_amd as pf
+from pocketforge_amd import weights as W
+
+pytestmark = pytest.mark.gpu
+
+CFG = {64: dict(n_layers=2, n_embd=1024, n_heads=16, head_dim=64, n_ff=512, n_vocab=1024, n_mtp=1),
+       128: dict(n_layers=2, n_embd=2048, n_heads=16, head_dim=128, n_ff=512, n_vocab=1024, n_mtp=1)}
+WIDE = dict(sink_size=4, window_size=2048, pool_block=16, max_context=2048)
+EDGE = dict(sink_size=4, window_size=500, pool_block=6, max_context=1024)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("kv,start,rows", [
+    (WIDE, 0, 9), (WIDE, 0, 97), (WIDE, 3, 128), (WIDE, 0, 256), (WIDE, 225, 97), (WIDE, 250, 256),
+    (WIDE, 1030, 16), (WIDE, 1030, 17), (WIDE, 1030, 31), (WIDE, 1055, 33), (WIDE, 1279, 65),
+    (EDGE, 400, 105), (EDGE, 400, 106), (dict(EDGE, sink_size=0), 0, 100), (dict(EDGE, sink_size=8), 1, 100),
+    (dict(EDGE, sink_size=9), 0, 100), (dict(EDGE, max_context=128), 29, 100), (dict(EDGE, max_context=128), 30, 100)])
+def test_tall_pass_equals_short_passes(gpu, hd, kv, start, rows):
+    cfg = CFG[hd]
+    m = pf.Model(gpu, cfg, W.make_weights(cfg, seed=5))
+    tall, short = pf.Engine(m, **kv), pf.Engine(m, **kv)
+    toks = W.prompt_ids(start + rows + 1, cfg["n_vocab"], seed=77)
+    for i in range(0, start, 8):
+        tall.prefill(toks[i:min(i + 8, start)])
+    tall.prefill(toks[start:start + rows])
+    for i in range(0, start + rows, 8):
+        short.prefill(toks[i:min(i + 8, start + rows)])
+    for head in range(cfg["n_heads"]):
+        a, b = (e.kv_export(0, 1, head, start + rows + 64) for e in (tall, short))
+        assert a[4] == b[4]
+        for x, y in zip(a[:4], b[:4]):
+            np.testing.assert_array_equal(x, y)
+    (la, ha), (lb, hb) = (e.forward(toks[start + rows:]) for e in (tall, short))
+    np.testing.assert_array_equal(ha, hb)
+    np.testing.assert_array_equal(la, lb)
+    tall.close()
+    short.close()
+    m.close()
