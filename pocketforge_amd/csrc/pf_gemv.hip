@@ -6,7 +6,7 @@
 //                  SiLU product in one launch.
 //  * row kernels   quantize_activation_row of whole rows, layer-skip
 //                  decisions and cache commits, embedding, small copies.
-//  * k_matmul_int8 / k_mm_epilogue: the reference's plain int8 matmul API.
+//  * k_matmul_i8   the reference's plain int8 matmul API.
 // The int8-activation x block-quantized products are in pf_mm.hip.
 #include "pf_device.h"
 
@@ -440,39 +440,102 @@ __global__ void k_embed(const uint8_t* __restrict__ codes, const uint16_t* __res
 
 // ============================================ reference plain-int8 matmul
 
-// C[i][j] = sum_k A[i][k] * B[j][k] (src/matmul_neon.cpp:80-144).  One
-// thread per output; K handled in 4-byte steps with an exact scalar tail.
-__global__ void k_matmul_int8(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
-                              int32_t* __restrict__ C, uint32_t M, uint32_t N, uint32_t K) {
-    uint32_t j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
-    if (j >= N || i >= M) return;
-    const int8_t* a = A + (size_t)i * K;
-    const int8_t* b = B + (size_t)j * K;
-    int acc = 0;
-    uint32_t k = 0;
-    if ((((uintptr_t)a | (uintptr_t)b) & 3u) == 0) {
-        for (; k + 4 <= K; k += 4)
-            acc = __builtin_amdgcn_sdot4(*reinterpret_cast<const int*>(a + k),
-                                         *reinterpret_cast<const int*>(b + k), acc, false);
+typedef int pf_i4 __attribute__((ext_vector_type(4)));
+typedef int pf_i16 __attribute__((ext_vector_type(16)));
+
+// 16 bytes k .. k + 15 of a row of K bytes at p (any alignment), zeros past
+// the row's end.
+__device__ __forceinline__ pf_i4 row_tail16(const int8_t* p, uint32_t k, uint32_t K) {
+    unsigned long long v[2] = {0ull, 0ull};
+    if (K >= 16u) {   // the row's last 16 bytes at most, moved down
+        const uint32_t o = min(k, K - 16u), sh = 8u * min(k - o, 16u);
+        __builtin_memcpy(v, p + o, 16);
+        if (sh >= 64u) {
+            v[0] = sh < 128u ? v[1] >> (sh - 64u) : 0ull;
+            v[1] = 0ull;
+        } else if (sh) {
+            v[0] = (v[0] >> sh) | (v[1] << (64u - sh));
+            v[1] >>= sh;
+        }
+    } else {
+        for (uint32_t i = 0; k + i < K; i++) {
+            const unsigned long long c = (unsigned long long)(uint8_t)p[k + i] << (8u * (i & 7u));
+            v[0] |= i < 8u ? c : 0ull;
+            v[1] |= i < 8u ? 0ull : c;
+        }
     }
-    for (; k < K; k++) acc += (int)a[k] * (int)b[k];
-    C[(size_t)i * N + j] = acc;
+    pf_i4 r;
+    __builtin_memcpy(&r, v, 16);
+    return r;
+}
+
+// C[i][j] = sum_k A[i][k] * B[j][k] (src/matmul_neon.cpp:80-144) on
+// v_mfma_i32_32x32x32_i8, any sizes and row alignments.  A workgroup of eight
+// waves owns 32 rows of A x 32 rows of B; wave w takes the 32-column steps
+// w, w + 8, ... of K with its operands straight from memory (16 bytes per
+// lane, four steps' loads together), and the waves' int32 sums meet in LDS
+// (exact, so the split changes nothing).  QUANT: the outputs leave as
+// (float)sum * as[i] * ws[j] (src/matmul_neon.cpp:176-180), else as int32.
+//
+// Latency bounds the API's sizes (a few MB): splitting K over the waves puts
+// most of a workgroup's loads into one round trip.  M 100, N 3000, K 1100:
+// 5.9 us beside 3.1 us for the row quantization, where one thread per output
+// took 332 us.  Workgroups of two or four A tiles (B read once for them)
+// measured the same at M 100-128 and slower at M = N / 16 = 256, K 4096
+// (four tiles 52.8 us, one 38.3).
+constexpr uint32_t MM_WAVES = 8;
+template <bool QUANT>
+__global__ __launch_bounds__(64 * MM_WAVES) void k_matmul_i8(const int8_t* __restrict__ A, uint32_t lda,
+                                                      const int8_t* __restrict__ B, uint32_t M, uint32_t N,
+                                                      uint32_t K, int32_t* __restrict__ Ci,
+                                                      const float* __restrict__ as, const float* __restrict__ ws,
+                                                      float* __restrict__ C) {
+    __shared__ int red[MM_WAVES][16][64];
+    constexpr uint32_t U = 4, W = MM_WAVES;
+    const uint32_t t = threadIdx.x, lane = t & 63u, r = lane & 31u, h = lane >> 5;
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t n0 = 32u * blockIdx.x, m0 = 32u * blockIdx.y;
+    const int8_t* bp = B + (size_t)min(n0 + r, N - 1u) * K;
+    const int8_t* ap = A + (size_t)min(m0 + r, M - 1u) * lda;
+    pf_i16 acc = {};
+    const uint32_t full = K >> 5;
+    for (uint32_t s0 = wid; s0 < full; s0 += U * W) {
+        pf_i4 a[U], b[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {   // past the last step: reloaded, not used
+            const uint32_t k = 32u * min(s0 + u * W, full - 1u) + 16u * h;
+            __builtin_memcpy(&b[u], bp + k, 16);
+            __builtin_memcpy(&a[u], ap + k, 16);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++)
+            if (s0 + u * W < full) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u], b[u], acc, 0, 0, 0);
+    }
+    if ((K & 31u) && wid == full % W) {
+        const uint32_t k = 32u * full + 16u * h;
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(row_tail16(ap, k, K), row_tail16(bp, k, K), acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 16; j++) red[wid][j][lane] = acc[j];
+    __syncthreads();
+    for (uint32_t x = t; x < 1024u; x += 64u * W) {
+        const uint32_t l = x & 63u, j = x >> 6;
+        const uint32_t m = m0 + 8u * (j >> 2) + 4u * (l >> 5) + (j & 3u), n = n0 + (l & 31u);
+        if (m >= M || n >= N) continue;
+        int v = red[0][j][l];
+#pragma unroll
+        for (uint32_t w = 1; w < W; w++) v += red[w][j][l];
+        if constexpr (QUANT) C[(size_t)m * N + n] = (float)v * as[m] * ws[n];
+        else Ci[(size_t)m * N + n] = v;
+    }
 }
 
 // matmul_quantized's given-scale activation path (src/matmul_neon.cpp:158-164).
 __global__ void k_quant_div(const float* __restrict__ A, const float* __restrict__ sc,
-                            int8_t* __restrict__ q, uint32_t M, uint32_t K) {
+                            int8_t* __restrict__ q, uint32_t q_stride, uint32_t M, uint32_t K) {
     uint32_t k = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
     if (k >= K || i >= M) return;
-    q[(size_t)i * K + k] = (int8_t)(int)__builtin_roundf(A[(size_t)i * K + k] / sc[i]);
-}
-
-// C = (float)C_int * a_scale[i] * w_scale[j] (src/matmul_neon.cpp:176-180).
-__global__ void k_mm_epilogue(const int32_t* __restrict__ Ci, const float* __restrict__ as,
-                              const float* __restrict__ ws, float* __restrict__ C, uint32_t M, uint32_t N) {
-    uint32_t j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
-    if (j >= N || i >= M) return;
-    C[(size_t)i * N + j] = (float)Ci[(size_t)i * N + j] * as[i] * ws[j];
+    q[(size_t)i * q_stride + k] = (int8_t)(int)__builtin_roundf(A[(size_t)i * K + k] / sc[i]);
 }
 
 }  // namespace pf

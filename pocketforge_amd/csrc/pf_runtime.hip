@@ -732,11 +732,18 @@ extern "C" pf_status pf_quantize_activation_rows(pf_ctx* c, const float* src, in
     return PF_OK;
 }
 
+template <bool QUANT>
+static void launch_matmul_i8(hipStream_t st, const int8_t* A, uint32_t lda, const int8_t* B, uint32_t M, uint32_t N,
+                             uint32_t K, int32_t* Ci, const float* as, const float* ws, float* C) {
+    hipLaunchKernelGGL(k_matmul_i8<QUANT>, dim3((N + 31) / 32, (M + 31) / 32), dim3(64 * MM_WAVES), 0, st, A, lda, B, M,
+                       N, K, Ci, as, ws, C);
+}
+
 extern "C" pf_status pf_matmul_int8(pf_ctx* c, const int8_t* A, const int8_t* B, int32_t* C, uint32_t M, uint32_t N,
                                     uint32_t K) {
     if (!c || !A || !B || !C) return PF_ERR_ARG;
     if (M == 0 || N == 0) return PF_OK;
-    hipLaunchKernelGGL(k_matmul_int8, dim3((N + 255) / 256, M), dim3(256), 0, c->stream, A, B, C, M, N, K);
+    launch_matmul_i8<false>(c->stream, A, K, B, M, N, K, C, nullptr, nullptr, nullptr);
     PF_LAUNCHED(c);
     return PF_OK;
 }
@@ -745,23 +752,21 @@ extern "C" pf_status pf_matmul_quantized(pf_ctx* c, const float* A, const int8_t
                                          uint32_t N, uint32_t K, const float* ws, const float* as_in) {
     if (!c || !A || !B || !C || !ws) return PF_ERR_ARG;
     if (M == 0 || N == 0) return PF_OK;
-    size_t need = (size_t)M * K + 256 + (size_t)M * 4 + 256 + (size_t)M * N * 4 + 256;
+    const uint32_t ldq = (K + 15u) / 16u * 16u;   // quantized rows start on 16 bytes
+    const size_t q_bytes = ((size_t)M * ldq + 255) & ~(size_t)255;
     void* s = nullptr;
-    pf_status st = ctx_scratch(c, need, &s);
+    pf_status st = ctx_scratch(c, q_bytes + (size_t)M * 4, &s);
     if (st) return st;
     int8_t* Aq = (int8_t*)s;
-    float* as = (float*)((char*)s + (((size_t)M * K + 255) & ~(size_t)255));
-    int32_t* Ci = (int32_t*)((char*)as + (((size_t)M * 4 + 255) & ~(size_t)255));
+    float* as = (float*)((char*)s + q_bytes);
     if (as_in) {
-        hipLaunchKernelGGL(k_quant_div, dim3((K + 255) / 256, M), dim3(256), 0, c->stream, A, as_in, Aq, M, K);
-        PF_HIP(c, hipMemcpyAsync(as, as_in, M * 4, hipMemcpyDeviceToDevice, c->stream));
+        hipLaunchKernelGGL(k_quant_div, dim3((K + 255) / 256, M), dim3(256), 0, c->stream, A, as_in, Aq, ldq, M, K);
     } else {
         if (!per_for(K)) return fail(c, PF_ERR_UNSUPPORTED, "K > 8192");
-        PF_PER_SWITCH(K, hipLaunchKernelGGL(k_quant_rows<PER>, dim3(M), dim3(256), 0, c->stream, A, K, K, Aq, K,
+        PF_PER_SWITCH(K, hipLaunchKernelGGL(k_quant_rows<PER>, dim3(M), dim3(256), 0, c->stream, A, K, K, Aq, ldq,
                                             as, (int32_t*)nullptr, 0u));
     }
-    hipLaunchKernelGGL(k_matmul_int8, dim3((N + 255) / 256, M), dim3(256), 0, c->stream, Aq, B, Ci, M, N, K);
-    hipLaunchKernelGGL(k_mm_epilogue, dim3((N + 255) / 256, M), dim3(256), 0, c->stream, Ci, as, ws, C, M, N);
+    launch_matmul_i8<true>(c->stream, Aq, ldq, B, M, N, K, nullptr, as_in ? as_in : as, ws, C);
     PF_LAUNCHED(c);
     return PF_OK;
 }

@@ -40,6 +40,32 @@ def test_quantize_activation_rows(gpu):
         assert s[m] == np.float32(s2)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (3, 33, 15), (1, 40, 16), (2, 31, 31), (33, 32, 33), (5, 77, 0),
+                                   (64, 65, 255), (31, 1000, 1100), (129, 4100, 47), (300, 4097, 130)])
+def test_matmul_i8_ragged(gpu, M, N, K):
+    """The MFMA int8 matmul at tile, step and row-tail edges and in each of
+    its tile shapes: integer sums equal, the scaled outputs bit for bit."""
+    rng = np.random.default_rng(M * 1000 + K)
+    A = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    B = rng.integers(-128, 128, (N, K), dtype=np.int8)
+    pad = lambda a: a if a.size else np.zeros(1, a.dtype)   # a buffer to point at
+    C = pf.DeviceArray.from_numpy(gpu, np.full((M, N), 7, np.int32))
+    a, b = _t(pad(A)), _t(pad(B))
+    gpu.check(pf.lib().pf_matmul_int8(gpu.h, a.ptr, b.ptr, C.ptr, M, N, K), "pf_matmul_int8")
+    gpu.synchronize()
+    np.testing.assert_array_equal(C.numpy(), A.astype(np.int32) @ B.astype(np.int32).T)
+    if K == 0:
+        return
+    Af = (rng.standard_normal((M, K)) * 0.5).astype(np.float32)
+    ws = (rng.random(N) * 0.02 + 0.001).astype(np.float32)
+    for act in (None, (np.abs(Af).max(1) / 120.0).astype(np.float32)):
+        ref = np.zeros((M, N), np.float32)
+        O.lib().orc_matmul_quantized(O.ptr(Af, O.f32p), O.ptr(B, O.i8p), O.ptr(ref, O.f32p), M, N, K,
+                                     O.ptr(ws, O.f32p), O.ptr(act, O.f32p) if act is not None else None)
+        got = gpu.matmul_quantized(_t(Af), _t(B), _t(ws), _t(act) if act is not None else None).numpy()
+        np.testing.assert_array_equal(got, ref)
+
+
 def test_matmul_int8_and_quantized(gpu):
     rng = np.random.default_rng(1)
     M, N, K = 5, 77, 300
