@@ -17,7 +17,10 @@ namespace pf {
 // The M activation rows (K <= 2048 floats each) staged once per workgroup
 // in LDS, then lane l's 32 elements of every row (block l) in registers
 // (zeros for lanes past the row's blocks): one copy of the rows per
-// workgroup from L2 instead of one per wave.
+// workgroup from L2 instead of one per wave.  Block b's 16-byte word i sits
+// at word i ^ ((b >> 1) & 7) of the block, so that 16 consecutive lanes
+// reading word i of their blocks fall on distinct banks (unswizzled, eight of
+// them share one: 18.9 against 15.0 us for 4 rows x a 16384 x 2048 matrix).
 template <int M>
 __device__ __forceinline__ void stage_rows(const float* __restrict__ h, uint32_t h_stride, uint32_t K, uint32_t lane,
                                            bool live, float (&hv)[M][32]) {
@@ -25,29 +28,82 @@ __device__ __forceinline__ void stage_rows(const float* __restrict__ h, uint32_t
     const uint32_t n4 = K >> 2;
     for (uint32_t i = threadIdx.x; i < M * n4; i += blockDim.x) {
         const uint32_t m = i / n4, c = i - m * n4;
-        reinterpret_cast<float4*>(hsm)[m * 512u + c] = *reinterpret_cast<const float4*>(h + (size_t)m * h_stride + 4u * c);
+        reinterpret_cast<float4*>(hsm)[m * 512u + (c ^ ((c >> 4) & 7u))] = *reinterpret_cast<const float4*>(h + (size_t)m * h_stride + 4u * c);
     }
     __syncthreads();
 #pragma unroll
     for (int m = 0; m < M; m++) {
 #pragma unroll
         for (int i = 0; i < 32; i += 4) {
-            const float4 v = live ? *reinterpret_cast<const float4*>(hsm + m * 2048 + lane * 32u + i)
+            const uint32_t w = ((uint32_t)i >> 2) ^ ((lane >> 1) & 7u);
+            const float4 v = live ? *reinterpret_cast<const float4*>(hsm + m * 2048 + lane * 32u + 4u * w)
                                   : make_float4(0.f, 0.f, 0.f, 0.f);
             hv[m][i] = v.x; hv[m][i + 1] = v.y; hv[m][i + 2] = v.z; hv[m][i + 3] = v.w;
         }
     }
 }
 
+// The 8 weights (nibble - 8) d of a Q4 code word in element order, each one
+// v_cvt_f32_ubyte and one v_fma (the asm keeps the compiler from extracting
+// the bytes first and from copying nd for a two-operand fma, which cost two
+// more steps per weight).
+__device__ __forceinline__ void q4_weights(uint32_t cw, float d, float nd, float (&w)[8]) {
+    uint32_t lo = cw & 0x0F0F0F0Fu, hi = (cw >> 4) & 0x0F0F0F0Fu;
+    asm("" : "+v"(lo), "+v"(hi));
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        const float x0 = (float)((lo >> (8 * b)) & 0xFFu), x1 = (float)((hi >> (8 * b)) & 0xFFu);
+        asm("v_fma_f32 %0, %1, %2, %3" : "=v"(w[2 * b]) : "v"(x0), "v"(d), "v"(nd));
+        asm("v_fma_f32 %0, %1, %2, %3" : "=v"(w[2 * b + 1]) : "v"(x1), "v"(d), "v"(nd));
+    }
+}
+
+// Halving trees of NV values per lane over the wave at once (wave_tree_sum's
+// order each): a level's pairs of values share one add, half of the lanes
+// summing one of them, down to the 8-lane level; the remaining levels run on
+// the ceil(NV / 8) words left.  On return lane l with l & 7 == 0 holds in
+// s[k] the sum of value 8 k + 4 (l >> 3 & 1) + 2 (l >> 4 & 1) + (l >> 5).
+// Against a tree of its own per value: 40 VALU steps instead of 224 (and no
+// LDS permutes) for 16 values.
+template <int NV>
+__device__ __forceinline__ void wave_tree_sums(const float (&v)[NV], float (&s)[(NV + 7) / 8]) {
+    constexpr int N1 = (NV + 1) / 2, N2 = (N1 + 1) / 2, N3 = (N2 + 1) / 2;
+    const uint32_t lane = threadIdx.x & 63u;
+    float a[N1], b[N2];
+#pragma unroll
+    for (int k = 0; k < N1; k++) {
+        const auto p = __builtin_amdgcn_permlane32_swap(f2u(v[2 * k]), f2u(v[2 * k + 1 < NV ? 2 * k + 1 : 2 * k]), false, false);
+        a[k] = u2f(p[0]) + u2f(p[1]);
+    }
+#pragma unroll
+    for (int k = 0; k < N2; k++) {
+        const auto p = __builtin_amdgcn_permlane16_swap(f2u(a[2 * k]), f2u(a[2 * k + 1 < N1 ? 2 * k + 1 : 2 * k]), false, false);
+        b[k] = u2f(p[0]) + u2f(p[1]);
+    }
+#pragma unroll
+    for (int k = 0; k < N3; k++) {
+        const float x = b[2 * k], y = b[2 * k + 1 < N2 ? 2 * k + 1 : 2 * k];
+        float t = ((lane & 8u) ? y : x) + dpp_mov<DPP_ROR8>((lane & 8u) ? x : y);
+        const float c = t + dpp_mov<DPP_ROR4>(t), d = t + dpp_mov<DPP_ROR12>(t);
+        t = (lane & 4u) ? c : d;
+        t = t + dpp_mov<DPP_XOR2>(t);
+        s[k] = t + dpp_mov<DPP_XOR1>(t);
+    }
+}
+
 // y[m][n] (+= y_in[m][n] when resid) = canonical fp32 dot of h[m] with row n:
 // lane l holds block l (K <= 2048), fmaf chain over the block's elements,
-// halving tree over the 64 lanes.  Each wave walks rows n = wave, wave +
-// total_waves, ..., loading the codes and scales of RB rows before their
-// products (the tied unembedding gives each wave 8 rows).  Grid y takes
-// the activation rows M at a time: slice y serves rows M y .. M y + M - 1.
+// halving tree over the 64 lanes.  Wave w walks the groups of RB rows
+// RB w, RB (w + total_waves), ..., loading a group's codes and scales before
+// its products.  Grid y takes the activation rows M at a time: slice y serves
+// rows M y .. M y + M - 1.
 // FMT: Q4 (16 code bytes per block: weight (nibble - 8) d, formed as
 // fmaf(nibble, d, -8 d), exact) or Q8 (32: weight (float)code * d, exact).
-template <int M, int FMT>
+// Bound: VALU issue (per 32 weights 72 steps to form them and 32 M fmaf, then
+// the trees).  16384 x 2048 Q4: 5.2 / 10.9 / 13.7 us for 1 / 4 / 5 rows; with
+// unswizzled staging, a tree of its own per sum and 4 + 1 rows in two launches
+// it took 7.1 / 18.8 / 25.1.
+template <int M, int FMT, int RB>
 __global__ __launch_bounds__(256) void k_gemv_f32(const uint8_t* __restrict__ codes,
                                                   const uint16_t* __restrict__ scales,
                                                   uint32_t N, uint32_t K,
@@ -64,14 +120,13 @@ __global__ __launch_bounds__(256) void k_gemv_f32(const uint8_t* __restrict__ co
     const bool live = lane < nb;
     float hv[M][32];
     stage_rows<M>(h, h_stride, K, lane, live, hv);
-    constexpr uint32_t RB = M == 1 ? 8u : (M <= 4 ? 4u : 2u);
-    for (uint32_t n0 = wave; n0 < N; n0 += RB * nwaves) {
+    for (uint32_t n0 = RB * wave; n0 < N; n0 += RB * nwaves) {
         constexpr uint32_t CB = FMT == FMT_Q8 ? 2u : 1u;   // 16-byte code words per block
         uint4 cr[RB][CB];
         float dr[RB];
 #pragma unroll
         for (uint32_t q = 0; q < RB; q++) {
-            const uint32_t n = n0 + q * nwaves;
+            const uint32_t n = n0 + q;
 #pragma unroll
             for (uint32_t u = 0; u < CB; u++) cr[q][u] = make_uint4(0u, 0u, 0u, 0u);
             dr[q] = 0.0f;
@@ -82,15 +137,13 @@ __global__ __launch_bounds__(256) void k_gemv_f32(const uint8_t* __restrict__ co
                 dr[q] = h2f(scales[(size_t)n * nb + lane]);
             }
         }
+        float acc[RB * M];   // value q M + m
 #pragma unroll
         for (uint32_t q = 0; q < RB; q++) {
-            const uint32_t n = n0 + q * nwaves;
-            if (n >= N) break;
-            float acc[M];
 #pragma unroll
-            for (int m = 0; m < M; m++) acc[m] = 0.0f;
+            for (int m = 0; m < M; m++) acc[q * M + m] = 0.0f;
             if (live) {
-                const float d = dr[q], nd = -8.0f * d;
+                const float d = dr[q];
                 if constexpr (FMT == FMT_Q8) {
                     const uint32_t cw[8] = {cr[q][0].x, cr[q][0].y, cr[q][0].z, cr[q][0].w,
                                             cr[q][1].x, cr[q][1].y, cr[q][1].z, cr[q][1].w};
@@ -98,30 +151,36 @@ __global__ __launch_bounds__(256) void k_gemv_f32(const uint8_t* __restrict__ co
                     for (int j = 0; j < 32; j++) {
                         const float wj = (float)(int8_t)((cw[j >> 2] >> (8 * (j & 3))) & 0xFFu) * d;
 #pragma unroll
-                        for (int m = 0; m < M; m++) acc[m] = __builtin_fmaf(hv[m][j], wj, acc[m]);
+                        for (int m = 0; m < M; m++) acc[q * M + m] = __builtin_fmaf(hv[m][j], wj, acc[q * M + m]);
                     }
                 } else {
                     const uint32_t cw[4] = {cr[q][0].x, cr[q][0].y, cr[q][0].z, cr[q][0].w};
+                    const float nd = -8.0f * d;
 #pragma unroll
-                    for (int j = 0; j < 16; j++) {
-                        uint32_t byte = (cw[j >> 2] >> (8 * (j & 3))) & 0xFFu;
-                        float w0 = __builtin_fmaf((float)(byte & 15u), d, nd);
-                        float w1 = __builtin_fmaf((float)(byte >> 4), d, nd);
+                    for (int i = 0; i < 4; i++) {
+                        float w[8];
+                        q4_weights(cw[i], d, nd, w);
 #pragma unroll
-                        for (int m = 0; m < M; m++) {
-                            acc[m] = __builtin_fmaf(hv[m][2 * j], w0, acc[m]);
-                            acc[m] = __builtin_fmaf(hv[m][2 * j + 1], w1, acc[m]);
-                        }
+                        for (int j = 0; j < 8; j++)
+#pragma unroll
+                            for (int m = 0; m < M; m++)
+                                acc[q * M + m] = __builtin_fmaf(hv[m][8 * i + j], w[j], acc[q * M + m]);
+                        // a word's weights at a time: all 32 cost 24 registers
+                        // and with them a wave per SIMD (4 rows)
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                 }
             }
+        }
+        float s[(RB * M + 7) / 8];
+        wave_tree_sums<RB * M>(acc, s);
 #pragma unroll
-            for (int m = 0; m < M; m++) {
-                float t = wave_tree_sum(acc[m]);
-                if (lane == 0) {
-                    size_t o = (size_t)m * y_stride + n;
-                    y[o] = y_in ? (y_in[o] + t) : t;
-                }
+        for (uint32_t k = 0; k < (RB * M + 7) / 8; k++) {
+            const uint32_t i = 8u * k + 4u * ((lane >> 3) & 1u) + 2u * ((lane >> 4) & 1u) + (lane >> 5);
+            const uint32_t n = n0 + i / M;
+            if ((lane & 7u) == 0 && i < RB * M && n < N) {
+                const size_t o = (size_t)(i % M) * y_stride + n;
+                y[o] = y_in ? (y_in[o] + s[k]) : s[k];
             }
         }
     }
@@ -156,20 +215,20 @@ __global__ __launch_bounds__(256) void k_gemv_f32_glu(const uint8_t* __restrict_
             const uint4 cg = *reinterpret_cast<const uint4*>(gcodes + ((size_t)n * nb + lane) * 16u);
             const uint4 cu = *reinterpret_cast<const uint4*>(ucodes + ((size_t)n * nb + lane) * 16u);
             const float dg = h2f(gscales[(size_t)n * nb + lane]), du = h2f(uscales[(size_t)n * nb + lane]);
-            const float ndg = -8.0f * dg, ndu = -8.0f * du;
             const uint32_t gw[4] = {cg.x, cg.y, cg.z, cg.w}, uw[4] = {cu.x, cu.y, cu.z, cu.w};
+            const float ndg = -8.0f * dg, ndu = -8.0f * du;
 #pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const uint32_t bg = (gw[j >> 2] >> (8 * (j & 3))) & 0xFFu, bu = (uw[j >> 2] >> (8 * (j & 3))) & 0xFFu;
-                const float g0 = __builtin_fmaf((float)(bg & 15u), dg, ndg), g1 = __builtin_fmaf((float)(bg >> 4), dg, ndg);
-                const float u0 = __builtin_fmaf((float)(bu & 15u), du, ndu), u1 = __builtin_fmaf((float)(bu >> 4), du, ndu);
+            for (int i = 0; i < 4; i++) {
+                float wg[8], wu[8];
+                q4_weights(gw[i], dg, ndg, wg);
+                q4_weights(uw[i], du, ndu, wu);
 #pragma unroll
-                for (int m = 0; m < M; m++) {
-                    ag[m] = __builtin_fmaf(hv[m][2 * j], g0, ag[m]);
-                    ag[m] = __builtin_fmaf(hv[m][2 * j + 1], g1, ag[m]);
-                    au[m] = __builtin_fmaf(hv[m][2 * j], u0, au[m]);
-                    au[m] = __builtin_fmaf(hv[m][2 * j + 1], u1, au[m]);
-                }
+                for (int j = 0; j < 8; j++)
+#pragma unroll
+                    for (int m = 0; m < M; m++) {
+                        ag[m] = __builtin_fmaf(hv[m][8 * i + j], wg[j], ag[m]);
+                        au[m] = __builtin_fmaf(hv[m][8 * i + j], wu[j], au[m]);
+                    }
             }
         }
 #pragma unroll

@@ -494,45 +494,66 @@ static void launch_gemm(hipStream_t st, const pf_matrix* W, MmKind kind, GemmArg
 constexpr uint32_t MAX_GEMM_ROWS = 512;
 static_assert(NOALLOC_SCALE_BYTES >= MAX_GEMM_ROWS * 4, "one scale per GEMM row");
 
-// y[m] (+= y_in[m]) = h[m] x dequantized rows, any M (launches of up to 8
-// rows; each row's result does not depend on the rows beside it).
-// Rows per slice of the fp32 GEMVs: 4 staged rows (128 VGPRs) leave room
-// for two waves per SIMD, where 8 rows (256 VGPRs) run one (64 sequences x
+// Rows per slice of the fp32 GEMVs in grid y: 4 staged rows (128 VGPRs) leave
+// room for two waves per SIMD, where 8 rows (256 VGPRs) run one (64 sequences x
 // 4 MTP heads: 49.2 -> 46.6 ms per round); the weights are read once per
 // slice, from L2.
 constexpr uint32_t F32_GROUP = 4;
 
+template <int M, int RB>
+static void gemv_f32_one(hipStream_t st, const pf_matrix* W, uint32_t slices, const float* h, uint32_t h_stride,
+                         float* y, uint32_t y_stride, const float* y_in, uint32_t max_waves) {
+    const uint32_t waves = std::min<uint32_t>((W->rows + RB - 1) / RB, max_waves);
+    const dim3 grid((waves + 3) / 4, slices);
+    if (W->fmt == FMT_Q8)
+        hipLaunchKernelGGL((k_gemv_f32<M, FMT_Q8, RB>), grid, dim3(256), 0, st, W->data, W->scales, W->rows, W->cols, h,
+                           h_stride, y, y_stride, y_in);
+    else
+        hipLaunchKernelGGL((k_gemv_f32<M, FMT_Q4, RB>), grid, dim3(256), 0, st, W->data, W->scales, W->rows, W->cols, h,
+                           h_stride, y, y_stride, y_in);
+}
+
+// Weight rows a wave takes together (their sums share one tree), so that the
+// matrix still makes 2048 waves: 4 (2 with more than 3 rows) from 8192 rows
+// on, 2 from 4096, else 1.  At 4096 rows, K 256 and 2 activation rows, 4 give
+// 4.5 us and 1 gives 4.9; at 2048 rows (a head) 1 stays at 3.9 us.
+template <int M>
+static void gemv_f32_rows(hipStream_t st, const pf_matrix* W, uint32_t slices, const float* h, uint32_t h_stride,
+                          float* y, uint32_t y_stride, const float* y_in, uint32_t max_waves) {
+    if (W->rows >= 8192)
+        gemv_f32_one<M, M <= 3 ? 4 : 2>(st, W, slices, h, h_stride, y, y_stride, y_in, max_waves);
+    else if (W->rows >= 4096)
+        gemv_f32_one<M, 2>(st, W, slices, h, h_stride, y, y_stride, y_in, max_waves);
+    else
+        gemv_f32_one<M, 1>(st, W, slices, h, h_stride, y, y_stride, y_in, max_waves);
+}
+
+// y[m] (+= y_in[m]) = h[m] x dequantized rows, any M (each row's result does
+// not depend on the rows beside it): 5 or 6 rows in one slice, else slices of
+// F32_GROUP rows in one launch and then the rest.
 static void launch_gemv_f32(hipStream_t st, const pf_matrix* W, uint32_t M, const float* h, uint32_t h_stride,
                             float* y, uint32_t y_stride, const float* y_in, uint32_t max_waves = 4096) {
-    uint32_t waves = std::min<uint32_t>(W->rows, max_waves);
-    // whole groups of F32_GROUP rows in one launch (grid y), then the rest
     constexpr uint32_t GR = F32_GROUP;
     for (uint32_t r0 = 0; r0 < M;) {
-        const uint32_t mb = std::min(GR, M - r0);
-        const dim3 grid((waves + 3) / 4, mb == GR ? (M - r0) / GR : 1u);
+        const uint32_t left = M - r0, mb = left == 5 || left == 6 ? left : std::min(GR, left);
+        const uint32_t slices = mb == GR ? left / GR : 1u;
         const float* hr = h + (size_t)r0 * h_stride;
         float* yr = y + (size_t)r0 * y_stride;
         const float* yi = y_in ? y_in + (size_t)r0 * y_stride : nullptr;
-#define PF_F32_CASE(MM)                                                                                       \
-    case MM:                                                                                                  \
-        if (W->fmt == FMT_Q8)                                                                                 \
-            hipLaunchKernelGGL((k_gemv_f32<MM, FMT_Q8>), grid, dim3(256), 0, st, W->data, W->scales, W->rows,   \
-                               W->cols, hr, h_stride, yr, y_stride, yi);                                      \
-        else                                                                                                  \
-            hipLaunchKernelGGL((k_gemv_f32<MM, FMT_Q4>), grid, dim3(256), 0, st, W->data, W->scales, W->rows,   \
-                               W->cols, hr, h_stride, yr, y_stride, yi);                                      \
-        break;
         switch (mb) {
-            PF_F32_CASE(1) PF_F32_CASE(2) PF_F32_CASE(3) PF_F32_CASE(4)
-            PF_F32_CASE(5) PF_F32_CASE(6) PF_F32_CASE(7) PF_F32_CASE(8)
+            case 1: gemv_f32_rows<1>(st, W, slices, hr, h_stride, yr, y_stride, yi, max_waves); break;
+            case 2: gemv_f32_rows<2>(st, W, slices, hr, h_stride, yr, y_stride, yi, max_waves); break;
+            case 3: gemv_f32_rows<3>(st, W, slices, hr, h_stride, yr, y_stride, yi, max_waves); break;
+            case 4: gemv_f32_rows<4>(st, W, slices, hr, h_stride, yr, y_stride, yi, max_waves); break;
+            case 5: gemv_f32_rows<5>(st, W, slices, hr, h_stride, yr, y_stride, yi, max_waves); break;
+            case 6: gemv_f32_rows<6>(st, W, slices, hr, h_stride, yr, y_stride, yi, max_waves); break;
         }
-#undef PF_F32_CASE
-        r0 += mb * grid.y;
+        r0 += mb * slices;
     }
 }
 
 // Gate and up products of one MTP head with the SiLU product fused:
-// a[m] = silu(Wg h[m]) * (Wu h[m]), rows in chunks of 8.
+// a[m] = silu(Wg h[m]) * (Wu h[m]), rows in slices of F32_GROUP.
 static void launch_gemv_f32_glu(hipStream_t st, const pf_matrix* Wg, const pf_matrix* Wu, uint32_t M, const float* h,
                                 uint32_t h_stride, float* a, uint32_t a_stride, uint32_t max_waves = 2048) {
     uint32_t waves = std::min<uint32_t>(Wg->rows, max_waves);
@@ -549,7 +570,6 @@ static void launch_gemv_f32_glu(hipStream_t st, const pf_matrix* Wg, const pf_ma
         break;
         switch (mb) {
             PF_GLU_CASE(1) PF_GLU_CASE(2) PF_GLU_CASE(3) PF_GLU_CASE(4)
-            PF_GLU_CASE(5) PF_GLU_CASE(6) PF_GLU_CASE(7) PF_GLU_CASE(8)
         }
 #undef PF_GLU_CASE
         r0 += mb * grid.y;

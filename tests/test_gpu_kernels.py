@@ -112,6 +112,22 @@ def test_gemv_int8_block(gpu, fmt, shape):
     W.close()
 
 
+@pytest.mark.parametrize("fmt", [pf.FMT_Q4, pf.FMT_Q8])
+@pytest.mark.parametrize("N,K", [(64, 256), (4032, 512), (4160, 768), (8192, 1024), (16384, 2048)])
+def test_gemv_f32_row_counts(gpu, N, K, fmt):
+    """1 to 8 activation rows (one slice of up to 6, else slices of 4) over
+    matrices on either side of the rows-per-wave thresholds."""
+    codes, scales = pf.gen_matrix(8, N, 0.02, N, K, fmt)
+    W = gpu.upload_matrix(fmt, codes, scales, rowmajor=True)
+    h = np.random.default_rng(N + K).standard_normal((8, K)).astype(np.float32)
+    ref = [O.gemv_f32(fmt, codes, scales, x) for x in h]
+    for M in range(1, 9):
+        y = gpu.gemv_f32(W, _t(h[:M])).numpy()
+        for m in range(M):
+            np.testing.assert_array_equal(y[m], ref[m], err_msg=f"{M} rows, row {m}")
+    W.close()
+
+
 def test_gemv_rejects_out_of_range_scales(gpu):
     codes, scales = pf.gen_matrix(5, 1, 0.02, 64, 256, pf.FMT_Q4)
     scales = scales.copy()
