@@ -1349,9 +1349,6 @@ __global__ __launch_bounds__(512) void k_attn_group(const PassDesc* __restrict__
 
 // ------------------------------------------------- row-tile attention
 
-typedef float pf_v16f __attribute__((ext_vector_type(16)));
-typedef float pf_v32f __attribute__((ext_vector_type(32)));
-
 // LDS of k_attn_tile (bytes): the tile's queries [hd / 4][32] float4
 // (swizzled) and the chunk's V rows [256][hd], reused for the sub-chunks'
 // partial sums [4][32][64]; then the V scales [256], the rows' sub-chunk

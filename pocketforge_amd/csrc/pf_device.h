@@ -14,6 +14,8 @@
 
 namespace pf {
 
+typedef float pf_v32f __attribute__((ext_vector_type(32)));
+
 __device__ __forceinline__ float u2f(uint32_t u) { return __uint_as_float(u); }
 __device__ __forceinline__ uint32_t f2u(float f) { return __float_as_uint(f); }
 

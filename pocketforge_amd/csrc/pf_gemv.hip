@@ -4,6 +4,8 @@
 //                  unembedding, MTP heads) in the canonical 64-lane order;
 //                  k_gemv_f32_glu: a head's gate and up products and their
 //                  SiLU product in one launch.
+//  * k_mm_f32      the same products of many activation rows on the fp32
+//                  matrix core.
 //  * row kernels   quantize_activation_row of whole rows, layer-skip
 //                  decisions and cache commits, embedding, small copies.
 //  * k_matmul_i8   the reference's plain int8 matmul API.
@@ -238,6 +240,180 @@ __global__ __launch_bounds__(256) void k_gemv_f32_glu(const uint8_t* __restrict_
                 const float sg = g / (1.0f + expf_c(-g));
                 a[(size_t)m * a_stride + n] = sg * u;
             }
+        }
+    }
+}
+
+// =========================================== fp32 x dequantized rows, tall
+
+// The canonical fp32 products of k_gemv_f32 (and with GLU the SiLU product of
+// k_gemv_f32_glu) for many activation rows, on v_mfma_f32_32x32x1_2b_f32: one
+// step of it rounds as one fmaf per element, so 32 steps over a 32-element
+// block are the block's fmaf chain bit for bit.  A wave owns 32 rows of h x 32
+// matrix rows; one step of its loop forms blocks l and l + 32 (the
+// instruction's two halves) and adds them, the halving tree's first level.
+// Blocks come in bit-reversed order of l, so the deeper levels join as a
+// binary counter of partial tiles.  KS > 1 splits the blocks over KS waves of
+// the workgroup by the tree's last levels, whose partial tiles meet in LDS.
+// Blocks past K / 32 count as zeros, as k_gemv_f32's idle lanes do.
+//
+// Grid 8 * mtiles * ceil(n groups / 8), a group being the 4 / KS matrix tiles
+// of a workgroup: workgroup b runs on XCD b mod 8, which so reads one eighth
+// of the matrix, each part for all the row tiles in turn.
+// What bounds it: fp32 issue (per 32 MFMAs of 32.8 ns, 72 steps to form the
+// weights and 32 adds of the tree do not overlap with them).  A 16384 x 2048
+// Q4 matrix takes 29 / 49 / 222 us for 32 / 64 / 320 rows (slices of 4 rows on
+// the VALU: 232 and 1130 for the last two), a head's gate, up and SiLU of 64
+// rows 30 (86), its down product 16 (45).
+// One wave per tile (KS 1) for more than 1024 tiles, else four.
+template <int FMT, bool GLU, int KS>
+__global__ __launch_bounds__(256, KS == 1 || GLU ? 2 : 3) void k_mm_f32(
+    const uint8_t* __restrict__ codes, const uint16_t* __restrict__ scales, const uint8_t* __restrict__ ucodes,
+    const uint16_t* __restrict__ uscales, uint32_t N, uint32_t K, uint32_t M, uint32_t mtiles,
+    const float* __restrict__ h, uint32_t h_stride, float* __restrict__ y, uint32_t y_stride,
+    const float* __restrict__ y_in) {
+    constexpr uint32_t NG = 4u / KS;                        // matrix tiles of a workgroup
+    constexpr uint32_t CB = FMT == FMT_Q8 ? 2u : 1u;        // 16-byte code words per block
+    constexpr int LV = KS == 1 ? 5 : (KS == 2 ? 4 : 3);     // tree levels inside the wave
+    __shared__ float red[KS > 1 ? 4 * 16 * 64 : 1];
+    const uint32_t t = threadIdx.x, lane = t & 63u, r = lane & 31u, hh = lane >> 5;
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(t >> 6), part = wid % KS;
+    const uint32_t slot = blockIdx.x >> 3, mt = slot % mtiles, grp = (slot / mtiles) * 8u + (blockIdx.x & 7u);
+    const uint32_t n0 = 32u * (grp * NG + wid / KS), m0 = 32u * mt, nb = K >> 5;
+    if (32u * grp * NG >= N) return;                        // the whole workgroup
+    const bool in = n0 < N;                                 // N % 64 == 0: whole tiles
+    const float* hr = h + (size_t)min(m0 + r, M - 1u) * h_stride;
+    const size_t wrow = (size_t)(in ? n0 + r : 0u) * nb;
+    constexpr uint32_t S = 32u / KS;
+    float tg[16], tot[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) tot[i] = tg[i] = 0.0f;
+#pragma unroll 1
+    for (uint32_t prod = 0; prod < (GLU ? 2u : 1u); prod++) {
+        const uint8_t* cp = GLU && prod ? ucodes : codes;
+        const uint16_t* sp = GLU && prod ? uscales : scales;
+        float st[LV][16];
+#pragma unroll
+        for (int k = 0; k < LV; k++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) st[k][i] = 0.0f;
+        // this lane's block of step s (clamped: loads past the blocks read the last)
+        auto blk = [&](uint32_t s) { return min((__brev(s) >> 27) + 32u * hh, nb - 1u); };
+        float4 a0[4], a1[4];
+        uint4 cw[CB];
+        uint32_t sc = 0;
+        uint32_t b = blk(part * S);
+#pragma unroll
+        for (int i = 0; i < 4; i++) a0[i] = *reinterpret_cast<const float4*>(hr + 32u * b + 4 * i);
+#pragma unroll
+        for (uint32_t u = 0; u < CB; u++) cw[u] = *reinterpret_cast<const uint4*>(cp + (wrow + b) * (16u * CB) + 16u * u);
+        sc = sp[wrow + b];
+#pragma unroll 1
+        for (uint32_t v = 0; v < S; v++) {
+            const uint32_t s = part * S + v, l = __brev(s) >> 27;
+            const uint32_t bn = blk(min(s + 1u, part * S + S - 1u));
+            const bool dead = l >= nb, half = l + 32u >= nb;     // no block at all, or none in the upper half
+            // the step's second half of h, and the next step's codes and first half
+#pragma unroll
+            for (int i = 0; i < 4; i++) a1[i] = *reinterpret_cast<const float4*>(hr + 32u * b + 16 + 4 * i);
+            uint4 cn[CB];
+#pragma unroll
+            for (uint32_t u = 0; u < CB; u++) cn[u] = *reinterpret_cast<const uint4*>(cp + (wrow + bn) * (16u * CB) + 16u * u);
+            const uint32_t sn = sp[wrow + bn];
+            const float d = h2f((uint16_t)sc), nd = -8.0f * d;
+            pf_v32f acc = {};
+            auto step8 = [&](int q, const float4 x, const float4 z) {   // elements 8 q .. 8 q + 7
+                float w[8];
+                if constexpr (FMT == FMT_Q8) {
+                    const uint4 c4 = cw[q >> 1];
+                    const uint32_t c0 = (q & 1) ? c4.z : c4.x, c1 = (q & 1) ? c4.w : c4.y;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        w[j] = (float)(int8_t)((c0 >> (8 * j)) & 0xFFu) * d;
+                        w[4 + j] = (float)(int8_t)((c1 >> (8 * j)) & 0xFFu) * d;
+                    }
+                } else {
+                    q4_weights(q == 0 ? cw[0].x : (q == 1 ? cw[0].y : (q == 2 ? cw[0].z : cw[0].w)), d, nd, w);
+                }
+                const float e[8] = {x.x, x.y, x.z, x.w, z.x, z.y, z.z, z.w};
+#pragma unroll
+                for (int j = 0; j < 8; j++) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(e[j], w[j], acc, 0, 0, 0);
+            };
+            auto clear_upper = [&](float4 (&a)[4]) {   // the missing block's lanes multiply zeros
+                if (!half) return;
+#pragma unroll
+                for (int i = 0; i < 4; i++) a[i] = hh ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : a[i];
+            };
+            if (!dead) {
+                clear_upper(a0);
+                step8(0, a0[0], a0[1]);
+                step8(1, a0[2], a0[3]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) a0[i] = *reinterpret_cast<const float4*>(hr + 32u * bn + 4 * i);
+            if (!dead) {
+                clear_upper(a1);
+                step8(2, a1[0], a1[1]);
+                step8(3, a1[2], a1[3]);
+            }
+            b = bn;
+            sc = sn;
+#pragma unroll
+            for (uint32_t u = 0; u < CB; u++) cw[u] = cn[u];
+            float x[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) x[i] = acc[i] + acc[16 + i];
+            // binary counter: level k waits in st[k] for its partner
+            bool carry = true;
+#pragma unroll
+            for (int k = 0; k < LV; k++) {
+                if (!carry) continue;
+                if ((v >> k) & 1u) {
+#pragma unroll
+                    for (int i = 0; i < 16; i++) x[i] = st[k][i] + x[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 16; i++) st[k][i] = x[i];
+                    carry = false;
+                }
+            }
+            if (v + 1u == S)
+#pragma unroll
+                for (int i = 0; i < 16; i++) tot[i] = x[i];
+        }
+        if constexpr (KS > 1) {
+            // parts in the counter's order: (0 + 1) + (2 + 3)
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 16; i++) red[(wid * 16u + i) * 64u + lane] = tot[i];
+            __syncthreads();
+            const uint32_t w0 = wid - part;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                float x = red[(w0 * 16u + i) * 64u + lane] + red[((w0 + 1u) * 16u + i) * 64u + lane];
+                if constexpr (KS == 4)
+                    x = x + (red[((w0 + 2u) * 16u + i) * 64u + lane] + red[((w0 + 3u) * 16u + i) * 64u + lane]);
+                tot[i] = x;
+            }
+        }
+        if (GLU && prod == 0)
+#pragma unroll
+            for (int i = 0; i < 16; i++) tg[i] = tot[i];
+    }
+    if (!in) return;
+    // register i: row m0 + 8 (i / 4) + 4 hh + i % 4, matrix row n0 + r; the
+    // parts share the tile's registers
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        if (i % KS != (int)part) continue;
+        const uint32_t m = m0 + 8u * (i / 4) + 4u * hh + (i % 4);
+        if (m >= M) continue;
+        const size_t o = (size_t)m * y_stride + n0 + r;
+        if constexpr (GLU) {
+            const float sg = tg[i] / (1.0f + expf_c(-tg[i]));
+            y[o] = sg * tot[i];
+        } else {
+            y[o] = y_in ? (y_in[o] + tot[i]) : tot[i];
         }
     }
 }

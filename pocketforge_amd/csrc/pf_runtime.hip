@@ -500,6 +500,35 @@ static_assert(NOALLOC_SCALE_BYTES >= MAX_GEMM_ROWS * 4, "one scale per GEMM row"
 // slice, from L2.
 constexpr uint32_t F32_GROUP = 4;
 
+// The same products (with Wu: their SiLU product) on the matrix core, from
+// where 32-row tiles beat slices of 4 rows (us at 8 / 12 / 16 / 20 rows): a
+// 16384 x 2048 matrix 21 / 30 / 38 / 46 against 28.9 for up to 32 rows, a 2048 x
+// 2048 one 9.0 / 10.6 / 14.4 / 17.6 against 15.8, its gate and up together 11.7 /
+// 14.6 / 18.9 / 21.9 against 30.
+static bool f32_tall(const pf_matrix* W, uint32_t M) { return M >= (W->rows >= 4096 ? 12u : 18u); }
+constexpr uint32_t GLU_TALL = 28;
+
+template <int FMT, bool GLU, int KS>
+static void mm_f32_one(hipStream_t st, const pf_matrix* W, const pf_matrix* Wu, uint32_t M, const float* h,
+                       uint32_t h_stride, float* y, uint32_t y_stride, const float* y_in) {
+    const uint32_t mtiles = (M + 31) / 32, groups = (W->rows / 32 + 4 / KS - 1) / (4 / KS);
+    hipLaunchKernelGGL((k_mm_f32<FMT, GLU, KS>), dim3(8 * mtiles * ((groups + 7) / 8)), dim3(256), 0, st, W->data,
+                       W->scales, Wu ? Wu->data : nullptr, Wu ? Wu->scales : nullptr, W->rows, W->cols, M, mtiles, h,
+                       h_stride, y, y_stride, y_in);
+}
+
+static void launch_mm_f32(hipStream_t st, const pf_matrix* W, uint32_t M, const float* h, uint32_t h_stride, float* y,
+                          uint32_t y_stride, const float* y_in) {
+    const bool split = (M + 31) / 32 * (W->rows / 32) <= 1024;   // tiles for one wave per SIMD, or fewer
+    if (W->fmt == FMT_Q8) {
+        if (split) mm_f32_one<FMT_Q8, false, 4>(st, W, nullptr, M, h, h_stride, y, y_stride, y_in);
+        else mm_f32_one<FMT_Q8, false, 1>(st, W, nullptr, M, h, h_stride, y, y_stride, y_in);
+    } else {
+        if (split) mm_f32_one<FMT_Q4, false, 4>(st, W, nullptr, M, h, h_stride, y, y_stride, y_in);
+        else mm_f32_one<FMT_Q4, false, 1>(st, W, nullptr, M, h, h_stride, y, y_stride, y_in);
+    }
+}
+
 template <int M, int RB>
 static void gemv_f32_one(hipStream_t st, const pf_matrix* W, uint32_t slices, const float* h, uint32_t h_stride,
                          float* y, uint32_t y_stride, const float* y_in, uint32_t max_waves) {
@@ -533,6 +562,7 @@ static void gemv_f32_rows(hipStream_t st, const pf_matrix* W, uint32_t slices, c
 // F32_GROUP rows in one launch and then the rest.
 static void launch_gemv_f32(hipStream_t st, const pf_matrix* W, uint32_t M, const float* h, uint32_t h_stride,
                             float* y, uint32_t y_stride, const float* y_in, uint32_t max_waves = 4096) {
+    if (f32_tall(W, M)) return launch_mm_f32(st, W, M, h, h_stride, y, y_stride, y_in);
     constexpr uint32_t GR = F32_GROUP;
     for (uint32_t r0 = 0; r0 < M;) {
         const uint32_t left = M - r0, mb = left == 5 || left == 6 ? left : std::min(GR, left);
@@ -556,6 +586,7 @@ static void launch_gemv_f32(hipStream_t st, const pf_matrix* W, uint32_t M, cons
 // a[m] = silu(Wg h[m]) * (Wu h[m]), rows in slices of F32_GROUP.
 static void launch_gemv_f32_glu(hipStream_t st, const pf_matrix* Wg, const pf_matrix* Wu, uint32_t M, const float* h,
                                 uint32_t h_stride, float* a, uint32_t a_stride, uint32_t max_waves = 2048) {
+    if (M >= GLU_TALL) return mm_f32_one<FMT_Q4, true, 4>(st, Wg, Wu, M, h, h_stride, a, a_stride, nullptr);
     uint32_t waves = std::min<uint32_t>(Wg->rows, max_waves);
     constexpr uint32_t GR = F32_GROUP;
     for (uint32_t r0 = 0; r0 < M;) {
