@@ -1678,7 +1678,7 @@ __global__ __launch_bounds__(128) void k_attn_merge_chunks(const PassDesc* __res
 // out = U * (1 / (T + 1e-10))), then the row quantized.  NT threads;
 // element i = t + NT k; heads * chunks <= 2048 (checked when the engine is
 // created).  fs and ts hold 2048 floats each, hmax and hinv 128, red 16.
-template <int PER, int NT>
+template <int PER, int NT, bool TILED>
 __device__ __forceinline__ void merge_quant_row(const PassDesc* __restrict__ pd, const KvGeom& g, uint32_t m,
                                                 const float* __restrict__ S, uint32_t s_stride,
                                                 const float* __restrict__ Up, uint32_t cstride,
@@ -1746,12 +1746,13 @@ __device__ __forceinline__ void merge_quant_row(const PassDesc* __restrict__ pd,
         const uint32_t i = t + (uint32_t)NT * k;
         v[k] = i < D ? v[k] * hinv[i / hd] : 0.0f;
     }
-    quantize_row_block<PER, NT>(v, D, q + (size_t)m * q_stride, as + m,
+    quantize_row_block<PER, NT, TILED>(v, D, q + (TILED ? operand_row(m, D) : (size_t)m * q_stride), as + m,
                                 bsum ? bsum + (size_t)m * bsum_stride : nullptr, red);
 }
 
-// Grid M + prefetch blocks, 1024 threads: merge_quant_row per row.
-template <int PER>
+// Grid M + prefetch blocks, 1024 threads: merge_quant_row per row; the codes
+// row-major (GEMV), or (TILED) in the GEMM's operand order.
+template <int PER, bool TILED>
 __global__ __launch_bounds__(1024) void k_attn_merge_quant(const PassDesc* __restrict__ pd, KvGeom g,
                                                            const float* __restrict__ S, uint32_t s_stride,
                                                            const float* __restrict__ Up, uint32_t cstride,
@@ -1767,7 +1768,7 @@ __global__ __launch_bounds__(1024) void k_attn_merge_quant(const PassDesc* __res
         return;
     }
     if (m >= pd->m) return;
-    merge_quant_row<PER, 1024>(pd, g, m, S, s_stride, Up, cstride, q, q_stride, as, bsum, bsum_stride, fs, ts,
+    merge_quant_row<PER, 1024, TILED>(pd, g, m, S, s_stride, Up, cstride, q, q_stride, as, bsum, bsum_stride, fs, ts,
                                       hmax, hinv, red);
 }
 

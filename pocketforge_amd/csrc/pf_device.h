@@ -331,11 +331,22 @@ __device__ __forceinline__ int half_wave_isum(int v) {
     return v;
 }
 
+// Offset of element i of a row in the GEMM's operand order: 32 rows' codes of
+// a 32-element block together, lane l = row + 32 (i % 32 / 16) of a wave
+// holding 16 bytes at 16 l (the MFMA operand), so a wave's load of a block is
+// one contiguous KiB.  Row m of K columns starts at (m / 32) 32 K + 16 (m %
+// 32).
+__device__ __forceinline__ uint32_t operand_off(uint32_t i) { return (i >> 5) * 1024u + (i & 16u) * 32u + (i & 15u); }
+__device__ __forceinline__ size_t operand_row(uint32_t m, uint32_t K) {
+    return (size_t)(m >> 5) * 32u * K + 16u * (m & 31u);
+}
+
 // Quantize one row held by a block of NT threads (thread t has elements
 // t, t+NT, ...) with the arithmetic of src/matmul_neon.cpp:16-29.  Writes
 // the codes, the row scale and (when bsum != null) the sums of the codes
 // of each 32-element block: a block's elements sit in 32 consecutive lanes.
-template <int PER, int NT>
+// TILED: the codes in operand order (q from operand_row).
+template <int PER, int NT, bool TILED = false>
 __device__ __forceinline__ void quantize_row_block(const float (&x)[PER], uint32_t K, int8_t* q,
                                                    float* scale_out, int32_t* bsum, float* red) {
     float amax = 0.0f;
@@ -352,7 +363,7 @@ __device__ __forceinline__ void quantize_row_block(const float (&x)[PER], uint32
         int code = 0;
         if (i < K) {
             int8_t c = quant_code(x[k], inv);
-            q[i] = c;
+            q[TILED ? operand_off(i) : i] = c;
             code = c;
         }
         if (bsum) {

@@ -514,7 +514,9 @@ __global__ __launch_bounds__(256) void k_rmsnorm_one(float* __restrict__ out, co
 
 // ============================================================ prologues
 
-template <int PER>
+// Rows quantized (quantize_activation_row): row-major with q_stride, or
+// (TILED) in the GEMM's operand order.
+template <int PER, bool TILED>
 __global__ __launch_bounds__(256) void k_quant_rows(const float* __restrict__ x, uint32_t x_stride,
                                                     uint32_t K, int8_t* __restrict__ q, uint32_t q_stride,
                                                     float* __restrict__ as, int32_t* __restrict__ bsum,
@@ -527,16 +529,15 @@ __global__ __launch_bounds__(256) void k_quant_rows(const float* __restrict__ x,
         uint32_t i = threadIdx.x + 256u * k;
         v[k] = i < K ? x[(size_t)m * x_stride + i] : 0.0f;
     }
-    quantize_row_block<PER, 256>(v, K, q + (size_t)m * q_stride, as + m,
+    quantize_row_block<PER, 256, TILED>(v, K, q + (TILED ? operand_row(m, K) : (size_t)m * q_stride), as + m,
                                  bsum ? bsum + (size_t)m * bsum_stride : nullptr, red);
 }
 
-// quantize_activation_row of rows of length K <= 1024 * PER, 1024 threads.
+// quantize_activation_row of rows of length K <= 1024 * PER into the GEMM's
+// operand order, 1024 threads.
 template <int PER>
 __global__ __launch_bounds__(1024) void k_quant_rows_wide(const float* __restrict__ x, uint32_t K,
-                                                          int8_t* __restrict__ q, uint32_t q_stride,
-                                                          float* __restrict__ as, int32_t* __restrict__ bsum,
-                                                          uint32_t bsum_stride) {
+                                                          int8_t* __restrict__ q, float* __restrict__ as) {
     __shared__ float red[16];
     const uint32_t m = blockIdx.x;
     float v[PER];
@@ -545,8 +546,7 @@ __global__ __launch_bounds__(1024) void k_quant_rows_wide(const float* __restric
         const uint32_t i = threadIdx.x + 1024u * k;
         v[k] = i < K ? x[(size_t)m * K + i] : 0.0f;
     }
-    quantize_row_block<PER, 1024>(v, K, q + (size_t)m * q_stride, as + m,
-                                  bsum ? bsum + (size_t)m * bsum_stride : nullptr, red);
+    quantize_row_block<PER, 1024, true>(v, K, q + operand_row(m, K), as + m, nullptr, red);
 }
 
 // LayerSkipController::should_skip_ffn (src/layer_skip.cpp:22-67) at one

@@ -12,8 +12,8 @@
 //            SwiGLU of interleaved gate/up rows).
 //  * k_gemm  M > 8 rows (prompt passes, many-sequence verify): the same
 //            exact arithmetic over 32-row activation tiles quantized by the
-//            row kernels, with the same epilogues; a workgroup shares each
-//            activation tile among its waves through LDS.
+//            row kernels, with the same epilogues; a workgroup's waves split
+//            K and meet in LDS.
 //
 // Arithmetic: v_mfma_i32_32x32x32_i8 gives the exact int32 dot p of one
 // 32-element block of an activation row and a weight row; the output is
@@ -787,171 +787,196 @@ __global__ __launch_bounds__(64 * GEMV_WAVES) void k_gemv(GemvArgs a) {
 struct GemmArgs {
     const uint8_t* W;
     uint32_t N, K, M;
-    const int8_t* act;         // [ceil(M / 32) * 32][act_stride] readable rows
-    uint32_t act_stride;
+    const int8_t* act;         // ceil(M / 32) * 32 rows in operand order (operand_off, pf_device.h)
     const float* as;           // [M]
     const uint32_t* gate;
     const uint8_t* xmin;       // [device rows]: smallest binade of the row's nonzero block scales
     MmEpi e;
 };
 
-// Integer form of a block scale for exact int64 sums: the fp16 scale d
-// (low 16 bits of h) is M * 2^(X - 25) with M = significand (hidden bit
-// included, 0 for zero) and X = max(biased exponent, 1); relative to the
-// row's smallest binade xmin (nonzero scales only, so X >= xmin whenever
-// M != 0) d = c * 2^(xmin - 25) with c = M << (X - xmin) < 2^26 (the
-// upload keeps nonzero scales of a row within 15 binades).
-__device__ __forceinline__ int32_t scale_multiplier(uint32_t h, uint32_t xmin) {
-    const uint32_t e = (h >> 10) & 31u, mt = h & 1023u;
-    const uint32_t mag = (e ? (mt | 1024u) : mt) << (((e ? e : 1u) - xmin) & 31u);
-    return (h & 0x8000u) ? -(int32_t)mag : (int32_t)mag;
-}
+// Integer form of a block scale for exact int64 sums: the fp16 scale d (low
+// 16 bits of h) is M * 2^(X - 25) with M = significand (hidden bit included, 0
+// for zero) and X = max(biased exponent, 1); relative to the row's smallest
+// binade xmin (nonzero scales only, so X >= xmin whenever M != 0) d = c *
+// 2^(xmin - 25) with c = M << (X - xmin) < 2^26 (the upload keeps nonzero
+// scales of a row within 15 binades).  c's 11 significant bits make d *
+// 2^(25 - xmin) exact in fp32.
+__device__ __forceinline__ int32_t scale_multiplier(uint32_t h, float up) { return (int32_t)(h2f((uint16_t)h) * up); }
 
-// One 256-column chunk of one wave's 32 x 32 output tile: eight blocks'
-// exact int32 dots (MFMA) times the blocks' integer scale multipliers into
-// int64 sums (|c p| < 2^41, so the sums of up to 8192 columns stay exact).
-// The MFMAs of DI blocks are issued before their products are added, so
-// the matrix core works while the adds of earlier blocks run.
-template <int FMT, int DI>
-__device__ __forceinline__ void gemm_chunk(int64_t (&S)[16], const uint8_t* arow, const uint4 (&cw)[sets_of<FMT>()],
-                                           const uint4& sw, uint32_t xmin) {
-    const pf_v16i zero = {};
-    pf_v4i A[8];
-#pragma unroll
-    for (uint32_t u = 0; u < 8; u++) A[u] = *reinterpret_cast<const pf_v4i*>(arow + 32u * u);
-    const uint32_t sx[4] = {sw.x, sw.y, sw.z, sw.w};
-#pragma unroll
-    for (uint32_t u0 = 0; u0 < 8; u0 += DI) {
-        pf_v16i D[DI];
-#pragma unroll
-        for (uint32_t j = 0; j < (uint32_t)DI; j++)
-            D[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[u0 + j], b_operand<FMT>(cw, u0 + j), zero, 0, 0, 0);
-#pragma unroll
-        for (uint32_t j = 0; j < (uint32_t)DI; j++) {
-            const uint32_t u = u0 + j;
-            const int32_t c = scale_multiplier(sx[u >> 1] >> (16u * (u & 1u)), xmin);
-#pragma unroll
-            for (int i = 0; i < 16; i++) S[i] += (int64_t)c * (int64_t)D[j][i];
-        }
+// Two blocks (64 columns) of one 32-row weight group for a lane: code words
+// and the two block scales.
+template <int FMT>
+struct GemmB {
+    uint32_t w[FMT == FMT_Q8 ? 8 : (FMT == FMT_Q4 ? 4 : 2)];
+    uint32_t sc;
+};
+
+// Step s (columns 64 s ..) of the group whose tiles start at `tiles`.
+template <int FMT>
+__device__ __forceinline__ void gemm_load_b(GemmB<FMT>& b, const uint8_t* tiles, uint32_t s, uint32_t lane) {
+    const uint8_t* tile = tiles + (size_t)(s >> 2) * g32_tile_bytes(FMT);
+    const uint32_t t = s & 3u;
+    if constexpr (FMT == FMT_Q8) {
+        const uint4 x = *reinterpret_cast<const uint4*>(tile + 2048u * t + 16u * lane);
+        const uint4 y = *reinterpret_cast<const uint4*>(tile + 2048u * t + 1024u + 16u * lane);
+        b.w[0] = x.x; b.w[1] = x.y; b.w[2] = x.z; b.w[3] = x.w;
+        b.w[4] = y.x; b.w[5] = y.y; b.w[6] = y.z; b.w[7] = y.w;
+    } else if constexpr (FMT == FMT_Q4) {
+        const uint4 x = *reinterpret_cast<const uint4*>(tile + 1024u * t + 16u * lane);
+        b.w[0] = x.x; b.w[1] = x.y; b.w[2] = x.z; b.w[3] = x.w;
+    } else {
+        const uint2 x = *reinterpret_cast<const uint2*>(tile + 1024u * (t >> 1) + 16u * lane + 8u * (t & 1u));
+        b.w[0] = x.x; b.w[1] = x.y;
     }
+    b.sc = *reinterpret_cast<const uint32_t*>(tile + g32_code_bytes(FMT) + 16u * (lane & 31u) + 4u * t);
 }
 
-// Grid (ceil(N / 32 / NW), ceil(M / 32 / MW)), 512 threads: 8 waves, wave
-// w takes M tile mw = w % MW (32 activation rows),
-// weight group nw = (w / MW) % NW of the workgroup's NW groups, and K slice
-// kw = w / (MW NW) (chunks c with c % KW == kw).  Step s covers chunks
-// KW s .. KW s + KW - 1: the workgroup copies their activation tiles
-// (32 MW rows x 256 B each) once into LDS (double buffer, rows padded to
-// 272 B) and every wave reads its rows from there, so a tile is fetched
-// once per workgroup instead of once per wave; one barrier per step.  Loads
-// run one step ahead (clamped, issued unconditionally), the weights into
-// two register sets used on alternate steps, so that no copy waits for
-// them.
-// K slices meet in LDS (exact int64 sums).  Two waves per SIMD (up to 256
-// VGPRs per lane): a 128-register budget spills.  Each lane keeps the 16
-// outputs of its MFMA tile as int64 multiples of its row's 2^(xmin - 25);
-// the epilogue converts them to fp64 exactly (|sum| < 2^53) and applies
-// y = (float)(sum * 2^(xmin - 25) * a_s), the value of the fp64 block sum.
-template <int MW, int KW>
-constexpr uint32_t gemm_smem() { return 2u * KW * 32u * MW * 272u; }
+// MFMA operand of block u (0, 1) of the step.  Q4 codes enter as 16 (nibble -
+// 8): the nibble with its top bit flipped is its two's complement, and in the
+// high half of a byte it needs no sign extension (two steps per four codes
+// fewer); gemm_shift takes the factor out of the sums.
+constexpr int gemm_shift(int fmt) { return fmt == FMT_Q4 ? 4 : 0; }
+template <int FMT>
+__device__ __forceinline__ pf_v4i gemm_operand(const GemmB<FMT>& b, uint32_t u) {
+    pf_v4i v;
+    if constexpr (FMT == FMT_Q8) {
+        v.x = (int)b.w[4 * u]; v.y = (int)b.w[4 * u + 1]; v.z = (int)b.w[4 * u + 2]; v.w = (int)b.w[4 * u + 3];
+    } else if constexpr (FMT == FMT_Q4) {
+        const uint32_t x0 = b.w[2 * u] ^ 0x88888888u, x1 = b.w[2 * u + 1] ^ 0x88888888u, mk = 0xF0F0F0F0u;
+        v.x = (int)((x0 << 4) & mk);
+        v.y = (int)((x1 << 4) & mk);
+        v.z = (int)(x0 & mk);
+        v.w = (int)(x1 & mk);
+    } else {
+        constexpr uint32_t ADD = (0x80u - (uint32_t)code_offset(FMT)) * 0x01010101u;
+        const uint32_t x = b.w[u], mk = 0x03030303u;
+        v.x = (int)(((x & mk) + ADD) ^ 0x80808080u);
+        v.y = (int)((((x >> 2) & mk) + ADD) ^ 0x80808080u);
+        v.z = (int)((((x >> 4) & mk) + ADD) ^ 0x80808080u);
+        v.w = (int)((((x >> 6) & mk) + ADD) ^ 0x80808080u);
+    }
+    return v;
+}
 
-template <int FMT, int EPI, bool GATED, int MW, int NW, int KW, int DI>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm(GemmArgs a) {
-    static_assert(MW * NW * KW == 8, "eight waves");
-    constexpr uint32_t TB = g32_tile_bytes(FMT), CODES = g32_code_bytes(FMT);
-    constexpr int SETS = sets_of<FMT>();
-    constexpr uint32_t ROWS = 32u * MW, AROW = 272u, STEP = KW * ROWS * AROW;
-    constexpr uint32_t APT = KW * MW;                  // 16-byte activation pieces per thread and step
-    static_assert((KW > 1 ? (KW - 1) * MW * NW * 64 * 16 * 8 : 0) <= 2 * STEP, "slice partials fit the buffers");
-    __shared__ __align__(16) uint8_t smem[2 * STEP];
+// A workgroup of KS waves owns 32 activation rows x 2 weight groups (64 device
+// rows); wave w takes the w-th share of the K / 64 steps.  Per step and lane
+// it loads its operands straight from memory (one step ahead, in two register
+// sets): two activation words (operand order, a contiguous KiB per wave), the
+// groups' codes and scales.  Each block's exact int32 dots (MFMA) times the
+// block's integer scale multiplier add into int64 sums (|c p| < 2^45 with Q4's
+// factor 16, so the sums of up to 8192 columns stay below 2^53).  The waves'
+// sums meet in LDS (exact), a few registers at a time, and each wave finishes
+// its share of the outputs: (float)(sum * 2^(xmin - 25) * a_s), the value of
+// the fp64 block sum.
+//
+// A block's MFMA (18 ns) costs about 27 VALU instructions, 16 of them the
+// v_mad_i64_i32 of its outputs (2.35 ns each), which bound the loop; at the
+// engine's sizes its start and end (a memory round trip each) count as much.
+// Four waves per SIMD hide them better than two of twice the rows, whose
+// shared operands save a quarter of the VALU work (25.4 against 25.2 us
+// below; 12.0 against 9.7 at 64 rows of 6144 x 2048).  Row-major activations
+// cost 32 segments per load (29.2 us).  Workgroup b runs on XCD b mod 8, which
+// so reads one eighth of the weights, each part for all the row tiles in turn.
+// With its row quantization, Q4, us at 32 / 256 / 512 rows: 6144 x 2048 9.4 /
+// 16.8 / 26.3, 11264 x 2048 9.7 / 25.2 / 40.8, 2048 x 2048 9.3 / 10.9 / 14.8,
+// 2048 x 5632 15.4 / 18.7 / 28.0; eight waves sharing row-major activation
+// tiles behind a barrier per 256 columns took 18.5 / 20.5 / 35.4, 18.6 / 34.7 /
+// 49.9, 13.0 / 14.2 / 15.4 and 24.6 / 26.9 / 29.8.
+template <int FMT, int EPI, bool GATED, int KS>
+__global__ __launch_bounds__(64 * KS, 4) void k_gemm(GemmArgs a) {
+    constexpr int NT = 2;
+    constexpr uint32_t PR = KS == 4 ? 8u : 4u;   // sum registers a wave hands over per phase (32 KB of LDS)
+    __shared__ __align__(16) int64_t red[KS][NT][PR][64];
     if constexpr (GATED)
         if (*a.gate == 0u) return;
     const uint32_t t = threadIdx.x, lane = t & 63u, r = lane & 31u, h = lane >> 5;
     const uint32_t wid = __builtin_amdgcn_readfirstlane(t >> 6);
-    const uint32_t mw = wid % MW, nw = (wid / MW) % NW, kw = wid / (MW * NW);
-    const uint32_t m0 = blockIdx.y * ROWS, ng = a.N >> 5, g = blockIdx.x * NW + nw, gc = min(g, ng - 1u);
-    const uint32_t nch = a.K >> 8, nsteps = (nch + KW - 1) / KW, mlast = a.M - 1u;
-    const uint8_t* tiles = a.W + (size_t)gc * nch * TB;
-    // piece u of thread t: row (t >> 4) + 32 (u % MW) of the tile, 16 bytes
-    // at 16 (t & 15) of chunk KW s + u / MW
-    const int8_t* abase[MW];
+    const uint32_t qn = a.N / 64u, qm = (a.M + 31u) / 32u, slot = blockIdx.x >> 3;
+    const uint32_t nq = (slot / qm) * 8u + (blockIdx.x & 7u), mt = slot % qm;
+    if (nq >= qn) return;
+    const uint32_t nch = a.K >> 8, ns = a.K >> 6;
+    const uint32_t s0 = ns * wid / KS, s1 = ns * (wid + 1u) / KS;
+    const uint8_t* tiles[NT];
+    float up[NT];
 #pragma unroll
-    for (uint32_t u = 0; u < (uint32_t)MW; u++)
-        abase[u] = a.act + (size_t)min(m0 + (t >> 4) + 32u * u, mlast) * a.act_stride + 16u * (t & 15u);
-    const uint32_t sbase = (t >> 4) * AROW + 16u * (t & 15u);
-    pf_v4i av[APT];
-#pragma unroll
-    for (uint32_t u = 0; u < APT; u++)
-        av[u] = *reinterpret_cast<const pf_v4i*>(abase[u % MW] + 256u * min(u / MW, nch - 1u));
-    uint4 cw0[SETS], cw1[SETS], sw0, sw1;
-    {
-        const uint8_t* tile = tiles + (size_t)min(kw, nch - 1u) * TB;
-#pragma unroll
-        for (int q = 0; q < SETS; q++) cw0[q] = *reinterpret_cast<const uint4*>(tile + q * 1024 + lane * 16);
-        sw0 = *reinterpret_cast<const uint4*>(tile + CODES + r * 16);
+    for (uint32_t n = 0; n < NT; n++) {
+        const uint32_t g = NT * nq + n;
+        tiles[n] = a.W + (size_t)g * nch * g32_tile_bytes(FMT);
+        up[n] = __builtin_amdgcn_ldexpf(1.0f, 25 - (int)a.xmin[32u * g + r]);
     }
-    int64_t S[16];
+    const int8_t* atile = a.act + (size_t)mt * 32u * a.K + 16u * lane;
+    int64_t S[NT][16];
 #pragma unroll
-    for (int i = 0; i < 16; i++) S[i] = 0;
-    const uint32_t xmin = a.xmin[32u * gc + r];
-    const uint32_t aoff = (kw * ROWS + 32u * mw + r) * AROW + 16u * h;
-    for (uint32_t st = 0; st < nsteps; st += 2) {
+    for (int n = 0; n < NT; n++)
 #pragma unroll
-        for (uint32_t ph = 0; ph < 2; ph++) {
-            const uint32_t s = st + ph;
-            if (ph == 1 && s >= nsteps) break;
-            uint8_t* buf = smem + ph * STEP;
+        for (int i = 0; i < 16; i++) S[n][i] = 0;
+    auto load = [&](pf_v4i (&A)[2], GemmB<FMT> (&B)[NT], uint32_t s) {
 #pragma unroll
-            for (uint32_t u = 0; u < APT; u++)
-                *reinterpret_cast<pf_v4i*>(buf + (u / MW) * ROWS * AROW + 32u * (u % MW) * AROW + sbase) = av[u];
-            __syncthreads();
-            const uint32_t nx = s + 1u < nsteps ? s + 1u : s;
-            const uint8_t* tile = tiles + (size_t)min(KW * nx + kw, nch - 1u) * TB;
-            // two register sets: step s uses set s & 1, the loads fill the other
+        for (uint32_t u = 0; u < 2; u++) A[u] = *reinterpret_cast<const pf_v4i*>(atile + 2048u * s + 1024u * u);
 #pragma unroll
-            for (int q = 0; q < SETS; q++) {
-                const uint4 w = *reinterpret_cast<const uint4*>(tile + q * 1024 + lane * 16);
-                if (ph == 0) cw1[q] = w; else cw0[q] = w;
+        for (uint32_t n = 0; n < NT; n++) gemm_load_b<FMT>(B[n], tiles[n], s, lane);
+    };
+    auto step = [&](const pf_v4i (&A)[2], const GemmB<FMT> (&B)[NT]) {
+        const pf_v16i zero = {};
+#pragma unroll
+        for (uint32_t u = 0; u < 2; u++)
+#pragma unroll
+            for (uint32_t n = 0; n < NT; n++) {
+                const int32_t c = scale_multiplier(B[n].sc >> (16u * u), up[n]);
+                const pf_v16i D = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[u], gemm_operand<FMT>(B[n], u), zero, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 16; i++) S[n][i] += (int64_t)c * (int64_t)D[i];
             }
-            const uint4 w = *reinterpret_cast<const uint4*>(tile + CODES + r * 16);
-            if (ph == 0) sw1 = w; else sw0 = w;
-#pragma unroll
-            for (uint32_t u = 0; u < APT; u++)
-                av[u] = *reinterpret_cast<const pf_v4i*>(abase[u % MW] + 256u * min(KW * nx + u / MW, nch - 1u));
-            if (KW * s + kw < nch) {
-                if (ph == 0) gemm_chunk<FMT, DI>(S, buf + aoff, cw0, sw0, xmin);
-                else gemm_chunk<FMT, DI>(S, buf + aoff, cw1, sw1, xmin);
-            }
+    };
+    if (s0 < s1) {
+        pf_v4i A0[2], A1[2];
+        GemmB<FMT> B0[NT], B1[NT];
+        load(A0, B0, s0);
+#pragma unroll 1
+        for (uint32_t s = s0; s < s1; s += 2) {
+            load(A1, B1, min(s + 1u, s1 - 1u));
+            step(A0, B0);
+            if (s + 1u >= s1) break;
+            load(A0, B0, min(s + 2u, s1 - 1u));
+            step(A1, B1);
         }
     }
-    if constexpr (KW > 1) {
-        int64_t* red = reinterpret_cast<int64_t*>(smem);   // [KW - 1][MW NW][16][64]: lanes on consecutive banks
-        __syncthreads();
-        if (kw > 0) {
+    // outputs: register i of lane (r, h) is activation row 8 (i / 4) + 4 h +
+    // i % 4 of the tile, device row r of its group.  Phase ph takes registers
+    // PR ph ..; wave w finishes words PP w .. of the phase's NT x PR
+    constexpr uint32_t NP = 16u / PR, PP = NT * PR / KS;
+    static_assert(PP <= PR, "a wave's words lie in one group");
+    const uint32_t tl = PP * wid / PR, jw = PP * wid % PR, mt0 = 32u * mt + 4u * h;
+    const uint32_t n = 32u * (NT * nq + tl) + r;
+    EpiPre pre[NP][PP];
+    float as[NP][PP];
+    asm volatile("" ::: "memory");   // the loads below stay behind the loop, whose registers they take
 #pragma unroll
-            for (int i = 0; i < 16; i++) red[(((kw - 1u) * MW * NW + mw + MW * nw) * 16u + i) * 64u + lane] = S[i];
+    for (uint32_t ph = 0; ph < NP; ph++)
+#pragma unroll
+        for (uint32_t k = 0; k < PP; k++) {
+            const uint32_t i = PR * ph + jw + k, m = min(mt0 + 8u * (i >> 2) + (i & 3u), a.M - 1u);
+            pre[ph][k] = epi_prefetch<EPI>(a.e, m, n);
+            as[ph][k] = a.as[m];
         }
+    const double unit = __builtin_ldexp(1.0, (int)a.xmin[n] - 25 - gemm_shift(FMT));
+#pragma unroll
+    for (uint32_t ph = 0; ph < NP; ph++) {
+        if (ph) __syncthreads();
+#pragma unroll
+        for (uint32_t g = 0; g < NT; g++)
+#pragma unroll
+            for (uint32_t j = 0; j < PR; j++) red[wid][g][j][lane] = S[g][PR * ph + j];
         __syncthreads();
-        if (kw == 0) {
 #pragma unroll
-            for (uint32_t k = 1; k < (uint32_t)KW; k++)
+        for (uint32_t k = 0; k < PP; k++) {
+            int64_t v = red[0][tl][jw + k][lane];
 #pragma unroll
-                for (int i = 0; i < 16; i++) S[i] += red[(((k - 1u) * MW * NW + mw + MW * nw) * 16u + i) * 64u + lane];
-        }
-    }
-    if (kw != 0u || g >= ng) return;   // whole waves
-    // output i of lane (r, h): activation row 8 (i / 4) + 4 h + i % 4 of the
-    // wave's M tile, device row r of group g
-    const uint32_t n = 32u * g + r;
-    const double unit = __builtin_ldexp(1.0, (int)xmin - 25);
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const uint32_t m = m0 + 32u * mw + 8u * (i / 4) + 4u * h + (i % 4);
-        const float y = m < a.M ? (float)(((double)S[i] * unit) * (double)a.as[m]) : 0.0f;
-        const float y1 = __shfl_xor(y, 1, 64), y16 = __shfl_xor(y, 16, 64);
-        if (m < a.M) {
-            const EpiPre pre = epi_prefetch<EPI>(a.e, m, n);
-            epi_apply<EPI>(a.e, pre, a.N, m, n, y, y1, y16);
+            for (uint32_t w = 1; w < KS; w++) v += red[w][tl][jw + k][lane];
+            const uint32_t i = PR * ph + jw + k, m = mt0 + 8u * (i >> 2) + (i & 3u);
+            const float y = (float)(((double)v * unit) * (double)as[ph][k]);
+            const float y1 = __shfl_xor(y, 1, 64), y16 = __shfl_xor(y, 16, 64);
+            if (m < a.M) epi_apply<EPI>(a.e, pre[ph][k], a.N, m, n, y, y1, y16);
         }
     }
 }
@@ -1017,12 +1042,12 @@ __global__ __launch_bounds__(1024) void k_norm_rows(const float* __restrict__ x,
     }
 }
 
-// Grid M, 1024 threads: normed rows quantized (quantize_activation_row)
-// into q [M][q_stride] with row scales as[M].
+// Grid M, 1024 threads: normed rows quantized (quantize_activation_row) into
+// q in the GEMM's operand order, with row scales as[M].
 template <int PER>
 __global__ __launch_bounds__(1024) void k_norm_quant(const float* __restrict__ x, uint32_t K,
                                                      const float* __restrict__ w, int8_t* __restrict__ q,
-                                                     uint32_t q_stride, float* __restrict__ as) {
+                                                     float* __restrict__ as) {
     __shared__ float row[4096];
     __shared__ float tree[64];
     __shared__ float red[16];
@@ -1036,7 +1061,7 @@ __global__ __launch_bounds__(1024) void k_norm_quant(const float* __restrict__ x
     }
     norm_row_1024<PER>(xv, wv, K, row, tree, red);
     __syncthreads();
-    quantize_row_block<PER, 1024>(xv, K, q + (size_t)m * q_stride, as + m, nullptr, red);
+    quantize_row_block<PER, 1024, true>(xv, K, q + operand_row(m, K), as + m, nullptr, red);
 }
 
 }  // namespace pf

@@ -426,22 +426,22 @@ static void gemv_cpw(hipStream_t st, const GemvArgs& a, hipEvent_t ev0, hipEvent
     else gemv_mr<F, PRO, EPI, G, 4>(st, a, ev0, ev1);
 }
 
-template <int F, int EPI, bool G, int MW, int NW, int KW, int DI>
-static void gemm_tiled(hipStream_t st, const GemmArgs& a, hipEvent_t ev0, hipEvent_t ev1) {
-    const dim3 grid((a.N / 32 + NW - 1) / NW, (a.M + 32 * MW - 1) / (32 * MW));
-    if (ev0) hipExtLaunchKernelGGL((k_gemm<F, EPI, G, MW, NW, KW, DI>), grid, dim3(512), 0, st, ev0, ev1, 0, a);
-    else hipLaunchKernelGGL((k_gemm<F, EPI, G, MW, NW, KW, DI>), grid, dim3(512), 0, st, a);
+template <int F, int EPI, bool G, int KS>
+static void gemm_split(hipStream_t st, const GemmArgs& a, hipEvent_t ev0, hipEvent_t ev1) {
+    const dim3 grid(8 * ((a.M + 31) / 32) * ((a.N / 64 + 7) / 8));
+    if (ev0) hipExtLaunchKernelGGL((k_gemm<F, EPI, G, KS>), grid, dim3(64 * KS), 0, st, ev0, ev1, 0, a);
+    else hipLaunchKernelGGL((k_gemm<F, EPI, G, KS>), grid, dim3(64 * KS), 0, st, a);
 }
 
-// Workgroup shapes measured at M = 320 on the 1B products: matrices of at
-// least 4096 rows take 32 activation rows x 8 row groups per workgroup;
-// narrower ones split K over two wave sets (32 x 4 x 2) so that the chip
-// still gets enough workgroups.  Every wave issues its chunk's 8 MFMAs
-// before their integer scaling.
+// K split over eight waves while the workgroups of that fit the chip about
+// once (two such workgroups per CU), else over four.  us with the row
+// quantization, 8 against 4 waves: 256 workgroups (256 rows of 2048 x 5632)
+// 18.7 / 22.8, 384 (128 rows of 6144 x 2048) 12.5 / 12.8, 704 (128 rows of
+// 11264 x 2048) 16.9 / 15.8, 1408 (256 rows) 27.1 / 25.2.
 template <int F, int EPI, bool G>
 static void gemm_one(hipStream_t st, const GemmArgs& a, hipEvent_t ev0, hipEvent_t ev1) {
-    if (a.N >= 4096) gemm_tiled<F, EPI, G, 1, 8, 1, 8>(st, a, ev0, ev1);
-    else gemm_tiled<F, EPI, G, 1, 4, 2, 8>(st, a, ev0, ev1);
+    if ((a.M + 31) / 32 * (a.N / 64) <= 512) gemm_split<F, EPI, G, 8>(st, a, ev0, ev1);
+    else gemm_split<F, EPI, G, 4>(st, a, ev0, ev1);
 }
 
 #define PF_MM_FMT(fmt, CALL)                                  \
@@ -649,17 +649,17 @@ static void launch_attn(hipStream_t st, uint32_t hd, uint32_t M, uint32_t tasks,
     // up to 256 workgroups, then 10 us per 256 more; k_attn_group's grows with
     // its blocks of 4 rows: 11.5 / 21 / 29 / 114 us at 192 / 384 / 576 / 2560 of
     // them (head_dim 128), 9 / 16 us at 16 / 192 (head_dim 64)
-    if (prefix && M > AG_MAX_ROWS && (M + 3) / 4 * tasks > (hd == 64 ? 192u : 384u)) {
+    if (prefix && !ev0 && M > AG_MAX_ROWS && (M + 3) / 4 * tasks > (hd == 64 ? 192u : 384u)) {
         // blocks b with equal b mod 8 (one XCD) hold whole (head, chunk)
         // groups of 32-row tiles
         const uint32_t tiles = (M + 31) / 32;
         const dim3 grid(8 * tiles * ((tasks + 7) / 8));
         if (hd == 64)
-            hipExtLaunchKernelGGL((k_attn_tile<4>), grid, dim3(256), 0, st, ev0, ev1, 0, pd, g, kv, l, M, tiles, tasks,
-                                  q, k, v, S, s_stride, Wp, cstride);
+            hipLaunchKernelGGL((k_attn_tile<4>), grid, dim3(256), 0, st, pd, g, kv, l, M, tiles, tasks, q, k, v, S,
+                               s_stride, Wp, cstride);
         else
-            hipExtLaunchKernelGGL((k_attn_tile<8>), grid, dim3(256), 0, st, ev0, ev1, 0, pd, g, kv, l, M, tiles, tasks,
-                                  q, k, v, S, s_stride, Wp, cstride);
+            hipLaunchKernelGGL((k_attn_tile<8>), grid, dim3(256), 0, st, pd, g, kv, l, M, tiles, tasks, q, k, v, S,
+                               s_stride, Wp, cstride);
         return;
     }
     if (batch && M > AG_MAX_ROWS && gsize >= 2 && gsize <= AS_NR) {
@@ -777,7 +777,7 @@ extern "C" pf_status pf_quantize_activation_rows(pf_ctx* c, const float* src, in
                                                  uint32_t M, uint32_t K) {
     if (!c || !src || !dst || !scales || M == 0) return PF_ERR_ARG;
     if (!per_for(K)) return fail(c, PF_ERR_UNSUPPORTED, "K > 8192");
-    PF_PER_SWITCH(K, hipLaunchKernelGGL(k_quant_rows<PER>, dim3(M), dim3(256), 0, c->stream, src, K, K, dst, K,
+    PF_PER_SWITCH(K, hipLaunchKernelGGL((k_quant_rows<PER, false>), dim3(M), dim3(256), 0, c->stream, src, K, K, dst, K,
                                         scales, (int32_t*)nullptr, 0u));
     PF_LAUNCHED(c);
     return PF_OK;
@@ -814,7 +814,7 @@ extern "C" pf_status pf_matmul_quantized(pf_ctx* c, const float* A, const int8_t
         hipLaunchKernelGGL(k_quant_div, dim3((K + 255) / 256, M), dim3(256), 0, c->stream, A, as_in, Aq, ldq, M, K);
     } else {
         if (!per_for(K)) return fail(c, PF_ERR_UNSUPPORTED, "K > 8192");
-        PF_PER_SWITCH(K, hipLaunchKernelGGL(k_quant_rows<PER>, dim3(M), dim3(256), 0, c->stream, A, K, K, Aq, ldq,
+        PF_PER_SWITCH(K, hipLaunchKernelGGL((k_quant_rows<PER, false>), dim3(M), dim3(256), 0, c->stream, A, K, K, Aq, ldq,
                                             as, (int32_t*)nullptr, 0u));
     }
     launch_matmul_i8<true>(c->stream, Aq, ldq, B, M, N, K, nullptr, as_in ? as_in : as, ws, C);
@@ -848,10 +848,10 @@ static pf_status gemv_q_run(pf_ctx* c, const pf_matrix* W, const float* x, float
         PF_LAUNCHED(c);
         return PF_OK;
     }
-    PF_PER_SWITCH(K, hipLaunchKernelGGL(k_quant_rows<PER>, dim3(M), dim3(256), 0, c->stream, x, K, K, act, K, as,
+    PF_PER_SWITCH(K, hipLaunchKernelGGL((k_quant_rows<PER, true>), dim3(M), dim3(256), 0, c->stream, x, K, K, act, K, as,
                                         (int32_t*)nullptr, 0u));
     GemmArgs g{};
-    g.W = W->data; g.N = N; g.K = K; g.M = M; g.act = act; g.act_stride = K; g.as = as; g.e = e;
+    g.W = W->data; g.N = N; g.K = K; g.M = M; g.act = act; g.as = as; g.e = e;
     launch_gemm(c->stream, W, MM_STORE, g);
     PF_LAUNCHED(c);
     return PF_OK;
@@ -1884,7 +1884,7 @@ static pf_status pass_mm(pf_engine* e, const pf_matrix* W, MmKind kind, uint32_t
     } else {
         GemmArgs g{};
         g.W = a.W; g.N = a.N; g.K = a.K; g.M = M;
-        g.act = e->act; g.act_stride = e->kmax; g.as = as_in; g.gate = a.gate; g.e = a.e;
+        g.act = e->act; g.as = as_in; g.gate = a.gate; g.e = a.e;
         launch_gemm(st, W, kind, g, ev0, ev1);
     }
     return PF_OK;
@@ -2214,7 +2214,7 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
         a.x = e->x; a.xs = D; a.nw = an;
         if (tall)
             PF_PER1024_SWITCH(D, hipLaunchKernelGGL(k_norm_quant<PER>, dim3(M), dim3(1024), 0, st, (const float*)e->x,
-                                                    D, an, e->act, ks, as0));
+                                                    D, an, e->act, as0));
         // passes of at most 8 rows: the QKV product and the attention in one
         // launch (its attention blocks load the cached K/V rows while the
         // product runs)
@@ -2332,11 +2332,19 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
             launch_attn(st, hd, M, attn_tasks, pd, g, e->kv, l, e->q, e->k, e->v, e->S, e->s_stride, e->Wp,
                         e->cstride, opf, batch, batch ? e->batch_group : 0u, prefix, aev0, aev1);
         }
-        if (!merge_in_o && !tail)
-            PF_PER1024_SWITCH(D, hipLaunchKernelGGL(k_attn_merge_quant<PER>, dim3(M + e->pf_blocks), dim3(1024), 0, st,
-                                                    pd, g, (const float*)e->S, e->s_stride, (const float*)e->Wp,
-                                                    e->cstride, e->act, ks, as1, (int32_t*)nullptr, 0u, M,
-                                                    prefetch_of(e, m->o[l], e->pf_blocks)));
+#define PF_MERGE(T)                                                                                                 \
+    PF_PER1024_SWITCH(D, hipLaunchKernelGGL((k_attn_merge_quant<PER, T>), dim3(M + e->pf_blocks), dim3(1024), 0, st, pd, \
+                                            g, (const float*)e->S, e->s_stride, (const float*)e->Wp, e->cstride,       \
+                                            e->act, ks, as1, (int32_t*)nullptr, 0u, M,                                 \
+                                            prefetch_of(e, m->o[l], e->pf_blocks)))
+        if (!merge_in_o && !tail) {
+            if (tall) {
+                PF_MERGE(true)
+            } else {
+                PF_MERGE(false)
+            }
+        }
+#undef PF_MERGE
         // decode passes without layer skip: the merge, O, gate|up and down in
         // one launch; LL words in llt: residual rows [M][D], SwiGLU rows
         // [M][F], merged attention rows [M][D]
@@ -2423,14 +2431,13 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
                 a.x = nout; a.xs = D; a.gate = e->skip_nrun + l;
                 if (tall)
                     PF_PER1024_SWITCH(D, hipLaunchKernelGGL(k_quant_rows_wide<PER>, dim3(M), dim3(1024), 0, st,
-                                                            (const float*)nout, D, e->act, ks, as2,
-                                                            (int32_t*)nullptr, 0u));
+                                                            (const float*)nout, D, e->act, as2));
                 if (pf_status s = pass_mm(e, m->gu[l], MM_GU_SKIP, M, a, as2)) return s;
             } else {
                 a.x = e->x; a.xs = D; a.nw = fn;
                 if (tall)
                     PF_PER1024_SWITCH(D, hipLaunchKernelGGL(k_norm_quant<PER>, dim3(M), dim3(1024), 0, st,
-                                                            (const float*)e->x, D, fn, e->act, ks, as2));
+                                                            (const float*)e->x, D, fn, e->act, as2));
                 if (pf_status s = pass_mm(e, m->gu[l], MM_GU, M, a, as2)) return s;
             }
         }
@@ -2448,7 +2455,7 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
         }
         if (tall)
             PF_PER1024_SWITCH(F, hipLaunchKernelGGL(k_quant_rows_wide<PER>, dim3(M), dim3(1024), 0, st,
-                                                    (const float*)e->sg, F, e->act, ks, as3, (int32_t*)nullptr, 0u));
+                                                    (const float*)e->sg, F, e->act, as3));
         if (pf_status s = pass_mm(e, m->down[l], e->skip_on ? MM_DOWN_SKIP : MM_DOWN, M, a, as3)) return s;
     }
     // every row of a pass counts for the skip caches except in verify passes,
