@@ -932,7 +932,8 @@ struct pf_mtp {
     uint32_t H = 0, D = 0, V = 0;
     std::vector<pf_matrix*> mats;     // [H][3]: gate, up, down (row-major Q4)
     float* table = nullptr;           // [V][D] fp32, or null
-    float *cur = nullptr, *g = nullptr, *u = nullptr, *a = nullptr, *logits = nullptr;
+    float* cur = nullptr;             // [H + 1][D]: the hidden input, then each head's state
+    float *a = nullptr, *logits = nullptr;
 };
 
 extern "C" void pf_mtp_destroy(pf_mtp* m) {
@@ -941,9 +942,7 @@ extern "C" void pf_mtp_destroy(pf_mtp* m) {
     (void)hipStreamSynchronize(c->stream);
     for (pf_matrix* M : m->mats) pf_matrix_free(M);
     dfree(c, m->table, (size_t)m->V * m->D * 4);
-    dfree(c, m->cur, (size_t)m->D * 4);
-    dfree(c, m->g, (size_t)m->D * 4);
-    dfree(c, m->u, (size_t)m->D * 4);
+    dfree(c, m->cur, (size_t)(m->H + 1) * m->D * 4);
     dfree(c, m->a, (size_t)m->D * 4);
     dfree(c, m->logits, (size_t)m->H * m->V * 4);
     delete m;
@@ -959,9 +958,7 @@ extern "C" pf_status pf_mtp_create(pf_ctx* c, uint32_t n_heads, uint32_t n_embd,
     m->mats.assign((size_t)n_heads * 3, nullptr);
     pf_status s = PF_OK;
     for (uint32_t i = 0; i < n_heads * 3 && !s; i++) s = matrix_alloc(c, FMT_Q4, n_embd, n_embd, true, &m->mats[i]);
-    if (!s) s = dalloc_t(c, &m->cur, n_embd);
-    if (!s) s = dalloc_t(c, &m->g, n_embd);
-    if (!s) s = dalloc_t(c, &m->u, n_embd);
+    if (!s) s = dalloc_t(c, &m->cur, (size_t)(n_heads + 1) * n_embd);
     if (!s) s = dalloc_t(c, &m->a, n_embd);
     if (!s) s = dalloc_t(c, &m->logits, (size_t)n_heads * n_vocab);
     if (s) { pf_mtp_destroy(m); return s; }
@@ -999,15 +996,25 @@ extern "C" pf_status pf_mtp_heads_forward(pf_mtp* m, const float* hidden, float*
     hipStream_t st = c->stream;
     const uint32_t D = m->D, V = m->V;
     PF_HIP(c, hipMemcpyAsync(m->cur, hidden, (size_t)D * 4, hipMemcpyHostToDevice, st));
+    // the heads' states first (head k + 1 needs head k's state, not its
+    // logits), then all their logits in one pass over the table
     for (uint32_t k = 0; k < m->H; k++) {            // src/mtp.cpp:63-127
-        launch_gemv_f32_glu(st, m->mats[k * 3 + 0], m->mats[k * 3 + 1], 1, m->cur, D, m->a, D);
-        launch_gemv_f32(st, m->mats[k * 3 + 2], 1, m->a, D, m->cur, D, m->cur);
+        const float* in = m->cur + (size_t)k * D;
+        launch_gemv_f32_glu(st, m->mats[k * 3 + 0], m->mats[k * 3 + 1], 1, in, D, m->a, D);
+        launch_gemv_f32(st, m->mats[k * 3 + 2], 1, m->a, D, m->cur + (size_t)(k + 1) * D, D, in);
+    }
+    for (uint32_t k = 0; k < m->H;) {
+        const uint32_t n = m->table ? std::min(4u, m->H - k) : 1u;
+        const float* h = m->cur + (size_t)(k + 1) * D;
         float* lk = m->logits + (size_t)k * V;
-        if (m->table)
-            hipLaunchKernelGGL(k_gemv_f32_dense<1>, dim3((std::min<uint32_t>(V, 2048) + 3) / 4), dim3(256), 0, st,
-                               (const float*)m->table, V, D, (const float*)m->cur, D, lk, V);
-        else
-            hipLaunchKernelGGL(k_mtp_placeholder, dim3((V + 255) / 256), dim3(256), 0, st, lk, V, k);
+        const dim3 grid((std::min<uint32_t>(V, 2048) + 3) / 4);
+        const float* E = m->table;
+        if (!E) hipLaunchKernelGGL(k_mtp_placeholder, dim3((V + 255) / 256), dim3(256), 0, st, lk, V, k);
+        else if (n == 4) hipLaunchKernelGGL(k_gemv_f32_dense<4>, grid, dim3(256), 0, st, E, V, D, h, D, lk, V);
+        else if (n == 3) hipLaunchKernelGGL(k_gemv_f32_dense<3>, grid, dim3(256), 0, st, E, V, D, h, D, lk, V);
+        else if (n == 2) hipLaunchKernelGGL(k_gemv_f32_dense<2>, grid, dim3(256), 0, st, E, V, D, h, D, lk, V);
+        else hipLaunchKernelGGL(k_gemv_f32_dense<1>, grid, dim3(256), 0, st, E, V, D, h, D, lk, V);
+        k += n;
     }
     PF_LAUNCHED(c);
     PF_HIP(c, hipMemcpyAsync(logits, m->logits, (size_t)m->H * V * 4, hipMemcpyDeviceToHost, st));

@@ -156,3 +156,45 @@ def test_batch_rejects_single_sequence_calls(gpu, tiny_weights):
     with pytest.raises(pf.PFError):
         pf.BatchEngine(m, 200, **KV)
     m.close()
+
+
+@pytest.mark.parametrize("fmt", [pf.FMT_Q4, pf.FMT_Q8])
+@pytest.mark.parametrize("n,d,vocab", [(12, 256, 4096), (18, 768, 1024), (33, 1280, 4160), (65, 256, 16384), (40, 2048, 1024)])
+def test_unembedding_of_many_rows(gpu, n, d, vocab, fmt):
+    """Logits of a batched pass (the fp32 matrix-core product: one wave per
+    tile and K split over four, tables of 8 to 64 blocks per row) equal the
+    few-row product, pinned to the oracle, of the pass's hidden rows."""
+    cfg = dict(n_layers=1, n_embd=d, n_heads=d // 64, head_dim=64, n_ff=512, n_vocab=vocab, n_mtp=1)
+    w = W.make_weights(cfg, seed=3)
+    codes, scales = pf.gen_matrix(12, d, 0.02, vocab, d, fmt)
+    w["emb"] = (fmt, codes, scales)
+    m = pf.Model(gpu, cfg, w)
+    b = pf.BatchEngine(m, n, **KV)
+    logits, hidden = b.forward_batch(np.arange(n), (np.arange(n, dtype=np.int32) * 7 % vocab)[:, None])
+    E = gpu.upload_matrix(fmt, codes, scales, rowmajor=True)
+    hidden, logits = hidden.reshape(n, d), logits.reshape(n, vocab)
+    for i in range(0, n, 8):
+        ref = gpu.gemv_f32(E, pf.DeviceArray.from_numpy(gpu, hidden[i:i + 8])).numpy()
+        np.testing.assert_array_equal(logits[i:i + 8], ref)
+    E.close()
+    b.close()
+    m.close()
+
+
+@pytest.mark.parametrize("n_seq", [17, 28, 33])
+def test_draft_heads_of_many_sequences(gpu, tiny_weights, n_seq):
+    """The heads' gate|up and down products on either side of their
+    matrix-core thresholds: tokens equal a single engine's."""
+    cfg, w = tiny_weights
+    m = pf.Model(gpu, cfg, _mix(w, 0.0005, 11))
+    b, e = pf.BatchEngine(m, n_seq, **KV), pf.Engine(m, **KV)
+    prompts = [W.prompt_ids(5 + s % 7, cfg["n_vocab"], seed=s) for s in range(n_seq)]
+    toks, res = b.generate_batch(prompts, 12, TOP_P, np.arange(n_seq, dtype=np.uint64) + 3)
+    for s in (0, n_seq // 2, n_seq - 1):
+        e.reset()
+        t1, r1 = e.generate(prompts[s], 12, TOP_P, s + 3)
+        np.testing.assert_array_equal(toks[s], t1)
+        assert res[s].mtp_accepted == r1.mtp_accepted
+    b.close()
+    e.close()
+    m.close()

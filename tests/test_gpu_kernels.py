@@ -304,6 +304,42 @@ def test_mtp_heads_standalone(gpu, with_table):
     m.close()
 
 
+@pytest.mark.parametrize("heads,d,V", [(1, 256, 1024), (2, 768, 515), (3, 512, 2049), (5, 2048, 777), (6, 256, 64)])
+def test_mtp_heads_counts(gpu, heads, d, V):
+    """Every slice height of the dense table pass (four heads, then the rest)
+    and vocabularies that do not fill its waves, bit-exact."""
+    m = pf.MTPHeads(gpu, heads, d, V)
+    ws = []
+    for k in range(heads):
+        trip = []
+        for w in range(3):
+            codes, scales = pf.gen_matrix(78, 100 + 3 * k + w, 0.02, d, d, pf.FMT_Q4)
+            m.set_head(k, w, codes, scales)
+            trip.append((O.Q4, codes, scales))
+        ws.append(trip)
+    rng = np.random.default_rng(heads + d)
+    table = (rng.standard_normal((V, d)) * 0.02).astype(np.float32)
+    m.set_table(table)
+    hidden = rng.standard_normal(d).astype(np.float32)
+    np.testing.assert_array_equal(m.forward(hidden), O.mtp_heads_forward(ws, d, V, table, hidden))
+    m.close()
+
+
+@pytest.mark.parametrize("fmt", [pf.FMT_Q4, pf.FMT_Q2, pf.FMT_Q15, pf.FMT_Q8])
+@pytest.mark.parametrize("M,N,K", [(9, 64, 256), (33, 2112, 768), (320, 4096, 512), (257, 4160, 256)])
+def test_gemm_splits(gpu, fmt, M, N, K):
+    """Both K splits of the GEMM (eight and four waves), fewer steps than
+    waves, a last row tile of one row and groups that do not fill the XCDs."""
+    codes, scales = pf.gen_matrix(97, fmt * 13 + N, 0.02, N, K, fmt)
+    W = gpu.upload_matrix(fmt, codes, scales)
+    x = (np.random.default_rng(M + K).standard_normal((M, K)) * 0.5).astype(np.float32)
+    y = gpu.gemv_q(W, _t(x)).numpy()
+    for m in sorted({0, 8, M // 2, M - 2, M - 1}):
+        a8, s = O.quantize_activation_row(x[m])
+        np.testing.assert_array_equal(y[m], O.gemv_i8(fmt, codes, scales, a8, s), err_msg=f"row {m}")
+    W.close()
+
+
 @pytest.mark.parametrize("fmt", [pf.FMT_Q4, pf.FMT_Q2, pf.FMT_Q15, pf.FMT_Q8])
 @pytest.mark.parametrize("shape", [(128, 512), (320, 2048), (64, 1792)])
 def test_gemm_int8_block(gpu, fmt, shape):
