@@ -25,12 +25,12 @@ extern "C" uint32_t pf_batch_position(const pf_engine* e, uint32_t seq) {
 }
 
 // Prompt passes of one sequence: consecutive positions in passes of up to
-// one window (at most 256 rows), exactly as pf_generate's prefill.
+// one window (at most 512 rows), exactly as pf_generate's prefill.
 static pf_status batch_prefill_seq(pf_engine* e, uint32_t seq, const int32_t* tokens, uint32_t n) {
     pf_ctx* c = e->c;
     hipStream_t st = c->stream;
-    for (uint32_t i = 0; i < n; i += e->prefill_rows) {
-        const uint32_t k = std::min(e->prefill_rows, n - i);
+    for (uint32_t i = 0, k; i < n; i += k) {
+        k = prompt_rows(e, e->spos[seq], n - i);
         e->pd_host.pos0 = e->spos[seq];
         e->pd_host.m = k;
         e->pd_host.batch = 0;

@@ -1398,7 +1398,6 @@ struct pf_engine {
     std::vector<std::pair<void*, size_t>> owned;
     // host mirrors
     uint32_t pos = 0;
-    uint32_t pool_rows_max = 1;
     bool hidden_valid = false;
     size_t max_memory = 0;
     uint32_t pf_blocks = 128;     // blocks of the attention merge that prefetch the O weights (PF_PREFETCH_BLOCKS)
@@ -1561,7 +1560,6 @@ static pf_status engine_create(pf_model* m, const pf_cache_desc* cd, uint32_t ns
         PF_HIP(c, hipMemcpy(e->rope_s, sn.data(), sn.size() * 4, hipMemcpyHostToDevice));
     }
     e->kmax = std::max(D, F);
-    e->pool_rows_max = (MAX_PREFILL_ROWS + e->g.pool_block - 1) / e->g.pool_block + 1;
     // prompt passes: at most one window of rows, so that every pooled row a
     // pass sees was folded from entries stored before the pass
     e->prefill_rows = std::min(PR, e->g.window);
@@ -2090,6 +2088,21 @@ static void launch_stack(hipStream_t st, int32_t fg, uint32_t hd, uint32_t nl, c
     else stack_fmt<FMT_Q2, FMT_Q15>(st, hd, nl, lw, a, b, ao, ag, ad, tasks, ev0, ev1);
 }
 
+// Positions up to which every row's list is a prefix of the next row's and
+// holds one entry per earlier position: every sink position stored, nothing
+// past max_context, the window not yet full (0 if the sink is too large).
+static uint32_t prefix_end(const KvGeom& g) {
+    return g.sink_size <= KV_SINK_ROWS ? std::min(g.max_context, g.sink_size + g.window) : 0u;
+}
+
+// Rows of the next prompt pass at position pos: one that starts before
+// prefix_end stops there, so that all of it can take the attention of prefix
+// lists.
+static uint32_t prompt_rows(const pf_engine* e, uint32_t pos, uint32_t left) {
+    const uint32_t n = std::min(e->prefill_rows, left), end = prefix_end(e->g);
+    return pos < end && pos + n - 1 > end ? end + 1 - pos : n;
+}
+
 // One forward pass of M rows (the PassDesc at `pd` holds positions and
 // tokens; pos0 is the host's copy of the first position).  hidden/logits
 // outputs are device [M][D] / [M][V]; either may be null.  A batched pass
@@ -2121,11 +2134,8 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
     const uint32_t ks = e->kmax;
     const bool tall = M > GEMV_MAX_M;
     const bool merge_in_o = M == 1 && D <= 2048;
-    // every row's list is a prefix of the last row's and holds one entry per
-    // earlier position: one sequence, every sink position stored, nothing past
-    // max_context, and the last row's window not yet full
-    const bool prefix = !batch && !e->capturing && g.sink_size <= KV_SINK_ROWS && pos_last <= g.max_context &&
-                        pos_last <= g.sink_size + g.window;
+    // every row's list a prefix of the last row's (prefix_end)
+    const bool prefix = !batch && !e->capturing && pos_last <= prefix_end(g);
     // activation scales [4][rows] of the tall passes' row kernels
     float* as0 = e->as;                   // attention-norm act
     float* as1 = e->as + e->rows;         // attention output act
@@ -2135,7 +2145,8 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
     // pooled rows the pass can see (folded from window entries still in the ring)
     // and the embedded rows, in one launch (k_pass_prep)
     {
-        const uint32_t n_pool = g.n_layers * g.n_heads * (batch ? M : e->pool_rows_max);
+        // (a pass of M positions evicts at most M entries)
+        const uint32_t n_pool = g.n_layers * g.n_heads * (batch ? M : (M + g.pool_block - 1) / g.pool_block);
         hipLaunchKernelGGL(k_pass_prep, dim3(n_pool + (D + 127) / 128 * M), dim3(128), 0, st, g, e->kv, pd, n_pool,
                            m->emb->data, m->emb->scales, d.n_vocab, D, e->x, e->ep, (int32_t)m->emb->fmt);
     }
@@ -2479,7 +2490,7 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
 extern "C" pf_status pf_forward(pf_engine* e, const int32_t* tokens, uint32_t n, float* logits, float* hidden) {
     if (!e || !tokens || n == 0) return PF_ERR_ARG;
     if (e->nseq != 1) return fail(e->c, PF_ERR_STATE, "multi-sequence engine: use pf_batch_forward");
-    if (n > ((logits || hidden) ? MAX_PASS_ROWS : e->prefill_rows))
+    if (n > ((logits || hidden) ? MAX_PASS_ROWS : std::min(MAX_FORWARD_ROWS, e->prefill_rows)))
         return fail(e->c, PF_ERR_ARG, "pass too tall: 8 rows with outputs, else one window up to 256 rows");
     if (e->pos + n > e->rope_pos) return fail(e->c, PF_ERR_CAPACITY, "position beyond the engine's max_context");
     pf_ctx* c = e->c;
@@ -2809,9 +2820,9 @@ extern "C" pf_status pf_generate(pf_engine* e, const int32_t* prompt, uint32_t n
     if (n_prompt) PF_HIP(c, hipMemcpyAsync(e->tokens, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice, st));
     auto t0 = std::chrono::steady_clock::now();
     // prefill (src/engine.cpp:286-290): every prompt token forwarded in order,
-    // in passes of up to one window (256 rows), whose GEMMs run on MFMA
-    for (uint32_t i = 0; i < n_prompt; i += e->prefill_rows) {
-        const uint32_t n = std::min(e->prefill_rows, n_prompt - i);
+    // in passes of up to one window (512 rows), whose GEMMs run on MFMA
+    for (uint32_t i = 0, n; i < n_prompt; i += n) {
+        n = prompt_rows(e, e->pos, n_prompt - i);
         e->pd_host.pos0 = e->pos;
         e->pd_host.m = n;
         for (uint32_t r = 0; r < n; r++) e->pd_host.tok[r] = prompt[i + r];

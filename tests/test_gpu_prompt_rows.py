@@ -45,3 +45,31 @@ def test_tall_pass_equals_short_passes(gpu, hd, kv, start, rows):
     tall.close()
     short.close()
     m.close()
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("kv,n", [(WIDE, 1100), (EDGE, 504), (EDGE, 505), (EDGE, 506), (EDGE, 900),
+                                  (dict(EDGE, sink_size=9), 600), (dict(EDGE, max_context=520), 515),
+                                  (dict(EDGE, window_size=64), 300)])
+def test_prompt_equals_short_passes(gpu, hd, kv, n):
+    """A whole prompt in passes of up to 512 rows, cut where the window fills,
+    leaves the cache and the next logits as passes of 8 rows do."""
+    cfg = CFG[hd]
+    m = pf.Model(gpu, cfg, W.make_weights(cfg, seed=6))
+    b, short = pf.BatchEngine(m, 1, **kv), pf.Engine(m, **kv)
+    toks = W.prompt_ids(n + 1, cfg["n_vocab"], seed=78)
+    b.prefill_seq(0, toks[:n])
+    for i in range(0, n, 8):
+        short.prefill(toks[i:min(i + 8, n)])
+    for head in (0, cfg["n_heads"] - 1):
+        x, y = (e.kv_export(0, 1, head, n + 64) for e in (b, short))
+        assert x[4] == y[4]
+        for p, q in zip(x[:4], y[:4]):
+            np.testing.assert_array_equal(p, q)
+    lb, hb = b.forward_batch([0], toks[None, n:])
+    ls, hs = short.forward(toks[n:])
+    np.testing.assert_array_equal(hb[0], hs)
+    np.testing.assert_array_equal(lb[0], ls)
+    b.close()
+    short.close()
+    m.close()
