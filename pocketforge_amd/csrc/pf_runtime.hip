@@ -464,15 +464,7 @@ static void launch_gemv(hipStream_t st, const pf_matrix* W, MmKind kind, const G
         case MM_GU_SKIP: PF_MM_FMT(W->fmt, (gemv_mr<F, PRO_QUANT, EPI_SWIGLU, true, 1>(st, a, ev0, ev1))) break;
         case MM_DOWN: PF_MM_FMT(W->fmt, (gemv_cpw<F, PRO_QPART, EPI_RESID, false>(st, a, ev0, ev1))) break;
         case MM_DOWN_SKIP: PF_MM_FMT(W->fmt, (gemv_cpw<F, PRO_QPART, EPI_RESID, true>(st, a, ev0, ev1))) break;
-        default:
-            PF_MM_FMT(W->fmt, ({
-                          const uint32_t cpw = (a.K / 256 + GEMV_WAVES - 1) / GEMV_WAVES;
-                          if (cpw <= 1) gemv_one<F, PRO_QUANT, EPI_STORE, false, 1, 8>(st, a, ev0, ev1);
-                          else if (cpw == 2) gemv_one<F, PRO_QUANT, EPI_STORE, false, 2, 8>(st, a, ev0, ev1);
-                          else if (cpw == 3) gemv_one<F, PRO_QUANT, EPI_STORE, false, 3, 8>(st, a, ev0, ev1);
-                          else gemv_one<F, PRO_QUANT, EPI_STORE, false, 4, 8>(st, a, ev0, ev1);
-                      }))
-            break;
+        default: PF_MM_FMT(W->fmt, (gemv_cpw<F, PRO_QUANT, EPI_STORE, false>(st, a, ev0, ev1))) break;
     }
 }
 

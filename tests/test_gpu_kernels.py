@@ -304,6 +304,25 @@ def test_mtp_heads_standalone(gpu, with_table):
     m.close()
 
 
+@pytest.mark.parametrize("fmt", [pf.FMT_Q4, pf.FMT_Q2, pf.FMT_Q15, pf.FMT_Q8])
+@pytest.mark.parametrize("N,K", [(64, 256), (64, 3840), (128, 5632), (64, 8192)])
+def test_gemv_rows_held(gpu, fmt, N, K):
+    """pf_gemv_q at every row count a launch holds (1, up to 5, up to 8) and
+    one to four chunks per wave."""
+    codes, scales = pf.gen_matrix(96, fmt * 17 + K, 0.02, N, K, fmt)
+    W = gpu.upload_matrix(fmt, codes, scales)
+    x = (np.random.default_rng(K).standard_normal((8, K)) * 0.5).astype(np.float32)
+    ref = []
+    for row in x:
+        a8, s = O.quantize_activation_row(row)
+        ref.append(O.gemv_i8(fmt, codes, scales, a8, s))
+    for M in (1, 2, 4, 5, 6, 8):
+        y = gpu.gemv_q(W, _t(x[:M])).numpy()
+        for m in range(M):
+            np.testing.assert_array_equal(y[m], ref[m], err_msg=f"{M} rows, row {m}")
+    W.close()
+
+
 @pytest.mark.parametrize("heads,d,V", [(1, 256, 1024), (2, 768, 515), (3, 512, 2049), (5, 2048, 777), (6, 256, 64)])
 def test_mtp_heads_counts(gpu, heads, d, V):
     """Every slice height of the dense table pass (four heads, then the rest)
