@@ -507,9 +507,8 @@ __global__ __launch_bounds__(256) void k_rmsnorm_one(float* __restrict__ out, co
 
 // ============================================================ prologues
 
-// Rows quantized (quantize_activation_row): row-major with q_stride, or
-// (TILED) in the GEMM's operand order.
-template <int PER, bool TILED>
+// Rows quantized (quantize_activation_row), row-major with q_stride.
+template <int PER>
 __global__ __launch_bounds__(256) void k_quant_rows(const float* __restrict__ x, uint32_t x_stride,
                                                     uint32_t K, int8_t* __restrict__ q, uint32_t q_stride,
                                                     float* __restrict__ as, int32_t* __restrict__ bsum,
@@ -522,7 +521,7 @@ __global__ __launch_bounds__(256) void k_quant_rows(const float* __restrict__ x,
         uint32_t i = threadIdx.x + 256u * k;
         v[k] = i < K ? x[(size_t)m * x_stride + i] : 0.0f;
     }
-    quantize_row_block<PER, 256, TILED>(v, K, q + (TILED ? operand_row(m, K) : (size_t)m * q_stride), as + m,
+    quantize_row_block<PER, 256>(v, K, q + (size_t)m * q_stride, as + m,
                                  bsum ? bsum + (size_t)m * bsum_stride : nullptr, red);
 }
 

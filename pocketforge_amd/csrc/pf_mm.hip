@@ -877,9 +877,9 @@ __device__ __forceinline__ pf_v4i gemm_operand(const GemmB<FMT>& b, uint32_t u) 
 // below; 12.0 against 9.7 at 64 rows of 6144 x 2048).  Row-major activations
 // cost 32 segments per load (29.2 us).  Workgroup b runs on XCD b mod 8, which
 // so reads one eighth of the weights, each part for all the row tiles in turn.
-// With its row quantization, Q4, us at 32 / 256 / 512 rows: 6144 x 2048 9.4 /
-// 16.8 / 26.3, 11264 x 2048 9.7 / 25.2 / 40.8, 2048 x 2048 9.3 / 10.9 / 14.8,
-// 2048 x 5632 15.4 / 18.7 / 28.0; eight waves sharing row-major activation
+// With its row quantization, Q4, us at 32 / 256 / 512 rows: 6144 x 2048 9.2 /
+// 16.7 / 26.7, 11264 x 2048 9.5 / 25.6 / 42.0, 2048 x 2048 9.1 / 10.7 / 14.8,
+// 2048 x 5632 14.3 / 17.7 / 27.1; eight waves sharing row-major activation
 // tiles behind a barrier per 256 columns took 18.5 / 20.5 / 35.4, 18.6 / 34.7 /
 // 49.9, 13.0 / 14.2 / 15.4 and 24.6 / 26.9 / 29.8.
 template <int FMT, int EPI, bool GATED, int KS>
