@@ -1356,6 +1356,50 @@ __global__ __launch_bounds__(512) void k_attn_group(const PassDesc* __restrict__
 __host__ __device__ constexpr uint32_t at_region(uint32_t hd) { return hd * 128u + 256u * hd > 32768u ? hd * 384u : 32768u; }
 __host__ __device__ constexpr uint32_t at_smem(uint32_t hd) { return at_region(hd) + (256u + 2u * 128u + 32u) * 4u; }
 
+// The V chains of one wave's sub-chunk on the VALU, entry by entry, with a
+// test of each row's list instead of a weight 0: 0 times an infinite or NaN
+// value is NaN, so a row must not multiply such an entry at or past its own
+// position.  Same steps, order and register layout as the matrix-core chains.
+// The weights s pass through wl (E = hd / 4 entries x 32 rows at a time); ve
+// and vc are the sub-chunk's V codes and scales in LDS, jb its first entry.
+template <int PARTS>
+__device__ __forceinline__ void attn_tile_v_rows(const pf_v32f& s, pf_v32f (&w)[PARTS / 4], float* wl, const uint8_t* ve,
+                                                 const float* vc, uint32_t jb, uint32_t p0, uint32_t r, uint32_t hh) {
+    constexpr uint32_t hd = 16 * PARTS, NT = hd / 64u, E = hd / 4u;
+    auto fence = [] {   // the wave's own LDS accesses, other lanes' included, in this order
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    };
+#pragma unroll
+    for (uint32_t e0 = 0; e0 < 64; e0 += E) {
+#pragma unroll
+        for (uint32_t i = 0; i < 32; i++) {
+            const uint32_t o = 32u * (i >> 4) + 8u * ((i >> 2) & 3u) + (i & 3u);
+            if (o / E == e0 / E) wl[32u * (o - e0 + 4u * hh) + r] = s[i];
+        }
+        fence();
+#pragma unroll 1
+        for (uint32_t o = e0; o < e0 + E; o++) {
+            float v[2][NT];
+#pragma unroll
+            for (uint32_t b = 0; b < 2; b++)
+#pragma unroll
+                for (uint32_t n = 0; n < NT; n++) v[b][n] = (float)(int8_t)ve[hd * o + NT * (r + 32u * b) + n] * vc[o];
+#pragma unroll
+            for (uint32_t i = 0; i < 16; i++) {
+                const uint32_t row = 8u * (i >> 2) + 4u * hh + (i & 3u);
+                const float e = wl[32u * (o - e0) + row];
+                if (jb + o >= p0 + row) continue;
+#pragma unroll
+                for (uint32_t b = 0; b < 2; b++)
+#pragma unroll
+                    for (uint32_t n = 0; n < NT; n++) w[n][16u * b + i] = __builtin_fmaf(e, v[b][n], w[n][16u * b + i]);
+            }
+        }
+        fence();
+    }
+}
+
 // Engine attention (the first stage above) of a prompt pass whose rows'
 // lists are plain prefixes: every row sees the positions before its own and
 // nothing has left the window (row at position p: C = p entries, entry j at
@@ -1549,28 +1593,33 @@ __global__ __launch_bounds__(256, 3) void k_attn_tile(const PassDesc* __restrict
     if (on) {
         const uint8_t* vl = lds_opaque(vt) + (size_t)64u * sub * hd + NT * lane;
         const float* vc = lds_opaque(vsc) + 64u * sub;
+        if (diag && __ballot(!(128.0f * fabsf(vs) < __builtin_inff()))) {
+            attn_tile_v_rows<PARTS>(s, w, reinterpret_cast<float*>(smem) + 8u * hd * sub, vt + (size_t)64u * sub * hd, vc, jb,
+                                    p0, r, hh);   // the queries' region is free
+        } else {
 #pragma unroll
-        for (uint32_t o = 0; o < 64; o += 8) {   // entries o .. o + 7: registers i0 .. i0 + 3, both halves
-            const uint32_t i0 = 16u * (o >> 5) + 4u * ((o >> 3) & 3u);
-            float e[8];
+            for (uint32_t o = 0; o < 64; o += 8) {   // entries o .. o + 7: registers i0 .. i0 + 3, both halves
+                const uint32_t i0 = 16u * (o >> 5) + 4u * ((o >> 3) & 3u);
+                float e[8];
 #pragma unroll
-            for (uint32_t u = 0; u < 4; u++) {
-                const auto pr = __builtin_amdgcn_permlane32_swap(f2u(s[i0 + u]), f2u(s[i0 + u]), false, false);
-                e[u] = u2f(pr[0]);
-                e[4 + u] = u2f(pr[1]);
+                for (uint32_t u = 0; u < 4; u++) {
+                    const auto pr = __builtin_amdgcn_permlane32_swap(f2u(s[i0 + u]), f2u(s[i0 + u]), false, false);
+                    e[u] = u2f(pr[0]);
+                    e[4 + u] = u2f(pr[1]);
+                }
+                const float4 c0 = *reinterpret_cast<const float4*>(vc + o), c1 = *reinterpret_cast<const float4*>(vc + o + 4u);
+                const float sc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+                uint32_t cd[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++)
+                    cd[u] = NT == 2u ? *reinterpret_cast<const uint16_t*>(vl + (size_t)(o + u) * hd) : vl[(size_t)(o + u) * hd];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++)
+#pragma unroll
+                    for (uint32_t n = 0; n < NT; n++)
+                        w[n] = __builtin_amdgcn_mfma_f32_32x32x1f32(e[u], (n ? cvt_i8_1(cd[u]) : cvt_i8_0(cd[u])) * sc[u], w[n], 0,
+                                                                    0, 0);
             }
-            const float4 c0 = *reinterpret_cast<const float4*>(vc + o), c1 = *reinterpret_cast<const float4*>(vc + o + 4u);
-            const float sc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-            uint32_t cd[8];
-#pragma unroll
-            for (uint32_t u = 0; u < 8; u++)
-                cd[u] = NT == 2u ? *reinterpret_cast<const uint16_t*>(vl + (size_t)(o + u) * hd) : vl[(size_t)(o + u) * hd];
-#pragma unroll
-            for (uint32_t u = 0; u < 8; u++)
-#pragma unroll
-                for (uint32_t n = 0; n < NT; n++)
-                    w[n] = __builtin_amdgcn_mfma_f32_32x32x1f32(e[u], (n ? cvt_i8_1(cd[u]) : cvt_i8_0(cd[u])) * sc[u], w[n], 0,
-                                                                0, 0);
         }
         if (diag) {
             // the rows whose self entry is here add their own value's term;

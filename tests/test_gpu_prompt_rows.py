@@ -73,3 +73,40 @@ def test_prompt_equals_short_passes(gpu, hd, kv, n):
     b.close()
     short.close()
     m.close()
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("at,rows", [(40, 128), (63, 128), (95, 97), (130, 256), (300, 400)])
+def test_overflowed_value_stays_out_of_earlier_rows(gpu, hd, at, rows):
+    """A token whose values overflow (infinite V scale) leaves every row
+    before it as it is without that token: layer 1's cache of those rows,
+    which holds layer 0's attention, is the same bit for bit."""
+    cfg = CFG[hd]
+    w = W.make_weights(cfg, seed=9)
+    big, usual = 7, 8
+    # channel 4 is 0 in every table row but `big`'s, where the first norm takes
+    # it to about 1e38, and the V matrix on to infinity
+    fmt, codes, scales = w["emb"]
+    codes = codes.copy()
+    codes[:, 0, 2] = (codes[:, 0, 2] & 0xF0) | 8
+    codes[big, 0, 2] |= 15
+    w["emb"] = (fmt, codes, scales)
+    w["attn_norm"] = w["attn_norm"].copy()
+    w["attn_norm"][0, 4] = 5e37
+    fmt, codes, scales = w["layers"][0]["wv"]
+    w["layers"][0]["wv"] = (fmt, codes, (scales.view(np.float16) * np.float16(1024)).view(np.uint16))
+    m = pf.Model(gpu, cfg, w)
+    toks = W.prompt_ids(rows, cfg["n_vocab"], seed=79)
+    toks[toks == big] = usual
+    planes = []
+    for t in (usual, big):
+        e = pf.BatchEngine(m, 1, **WIDE)
+        toks[at] = t
+        e.prefill_seq(0, toks)
+        planes.append([[e.kv_export(0, layer, head, rows + 64)[:4] for head in (0, cfg["n_heads"] - 1)] for layer in (0, 1)])
+        e.close()
+    m.close()
+    for head in range(2):
+        assert np.isfinite(planes[0][1][head][3]).all() and not np.isfinite(planes[1][0][head][3][at])
+        for x, y in zip(planes[0][1][head], planes[1][1][head]):
+            np.testing.assert_array_equal(x[:at], y[:at])
