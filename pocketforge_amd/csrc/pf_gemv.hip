@@ -670,12 +670,17 @@ __global__ void k_embed(const uint8_t* __restrict__ codes, const uint16_t* __res
 typedef int pf_i4 __attribute__((ext_vector_type(4)));
 typedef int pf_i16 __attribute__((ext_vector_type(16)));
 
-// 16 bytes k .. k + 15 of a row of K bytes at p (any alignment), zeros past
-// the row's end.
-__device__ __forceinline__ pf_i4 row_tail16(const int8_t* p, uint32_t k, uint32_t K) {
+// Bytes k .. k + 15 of the K-byte row at offset `row` of a matrix of `total`
+// bytes at p (any alignment), zeros past the row's end: one 16-byte load, no
+// further than the row's end (K >= 16) or the matrix's, moved down into place.
+// (Rows of 4 to 12 bytes taken byte by byte cost up to 1.5 times the rest of a
+// 4096 x 4096 product.)
+__device__ __forceinline__ pf_i4 tail16(const int8_t* p, size_t total, size_t row, uint32_t k, uint32_t K) {
     unsigned long long v[2] = {0ull, 0ull};
-    if (K >= 16u) {   // the row's last 16 bytes at most, moved down
-        const uint32_t o = min(k, K - 16u), sh = 8u * min(k - o, 16u);
+    if (total >= 16u) {
+        const uint32_t kl = K >= 16u ? min(k, K - 16u) : 0u;
+        const size_t o = K >= 16u ? row + kl : min(row, total - 16u);
+        const uint32_t sh = 8u * min((uint32_t)(row - o) + k, 16u);
         __builtin_memcpy(v, p + o, 16);
         if (sh >= 64u) {
             v[0] = sh < 128u ? v[1] >> (sh - 64u) : 0ull;
@@ -684,9 +689,13 @@ __device__ __forceinline__ pf_i4 row_tail16(const int8_t* p, uint32_t k, uint32_
             v[0] = (v[0] >> sh) | (v[1] << (64u - sh));
             v[1] >>= sh;
         }
+        if (K < 16u) {   // k is 0 (the row) or 16 (all zeros)
+            v[0] = K >= 8u ? v[0] : v[0] & ((1ull << (8u * K)) - 1ull);
+            v[1] = K > 8u ? v[1] & ((1ull << (8u * K - 64u)) - 1ull) : 0ull;
+        }
     } else {
         for (uint32_t i = 0; k + i < K; i++) {
-            const unsigned long long c = (unsigned long long)(uint8_t)p[k + i] << (8u * (i & 7u));
+            const unsigned long long c = (unsigned long long)(uint8_t)p[row + k + i] << (8u * (i & 7u));
             v[0] |= i < 8u ? c : 0ull;
             v[1] |= i < 8u ? 0ull : c;
         }
@@ -697,36 +706,43 @@ __device__ __forceinline__ pf_i4 row_tail16(const int8_t* p, uint32_t k, uint32_
 }
 
 // C[i][j] = sum_k A[i][k] * B[j][k] (src/matmul_neon.cpp:80-144) on
-// v_mfma_i32_32x32x32_i8, any sizes and row alignments.  A workgroup of eight
-// waves owns 32 rows of A x 32 rows of B; wave w takes the 32-column steps
-// w, w + 8, ... of K with its operands straight from memory (16 bytes per
-// lane, four steps' loads together), and the waves' int32 sums meet in LDS
-// (exact, so the split changes nothing).  QUANT: the outputs leave as
-// (float)sum * as[i] * ws[j] (src/matmul_neon.cpp:176-180), else as int32.
+// v_mfma_i32_32x32x32_i8, any sizes and row alignments.  W waves own 32 rows
+// of A x 32 rows of B; wave w of them takes the 32-column steps w, w + W, ...
+// of K with its operands straight from memory (16 bytes per lane, four steps'
+// loads together), and their int32 sums meet in LDS (exact, so the split
+// changes nothing).  QUANT: the outputs leave as (float)sum * as[i] * ws[j]
+// (src/matmul_neon.cpp:176-180), else as int32.
 //
 // Latency bounds the API's sizes (a few MB): splitting K over the waves puts
 // most of a workgroup's loads into one round trip.  M 100, N 3000, K 1100:
 // 5.9 us beside 3.1 us for the row quantization, where one thread per output
 // took 332 us.  Workgroups of two or four A tiles (B read once for them)
 // measured the same at M 100-128 and slower at M = N / 16 = 256, K 4096
-// (four tiles 52.8 us, one 38.3).
+// (four tiles 52.8 us, one 38.3).  MM_SHORT_K columns or fewer are one round
+// trip for a wave alone, and from MM_SHORT_TILES tiles (eight waves per CU) on
+// the outputs are what counts: a tile per wave (W 1), stored from registers.
+// M 4096, N 4096, K 4: 14.1 us (W 8: 26.8); M 4096, N 16 (128 tiles) stays at
+// 7.4 us where W 1 takes 8.7.
 constexpr uint32_t MM_WAVES = 8;
-template <bool QUANT>
+constexpr uint32_t MM_SHORT_K = 128, MM_SHORT_TILES = 2048;
+template <bool QUANT, uint32_t W>
 __global__ __launch_bounds__(64 * MM_WAVES) void k_matmul_i8(const int8_t* __restrict__ A, uint32_t lda,
                                                       const int8_t* __restrict__ B, uint32_t M, uint32_t N,
                                                       uint32_t K, int32_t* __restrict__ Ci,
                                                       const float* __restrict__ as, const float* __restrict__ ws,
                                                       float* __restrict__ C) {
-    __shared__ int red[MM_WAVES][16][64];
-    constexpr uint32_t U = 4, W = MM_WAVES;
+    static_assert(W == 1 || W == MM_WAVES, "a tile per wave or per workgroup");
+    __shared__ int red[W][16][64];
+    constexpr uint32_t U = 4;
     const uint32_t t = threadIdx.x, lane = t & 63u, r = lane & 31u, h = lane >> 5;
-    const uint32_t wid = __builtin_amdgcn_readfirstlane(t >> 6);
-    const uint32_t n0 = 32u * blockIdx.x, m0 = 32u * blockIdx.y;
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(t >> 6), part = W == 1u ? 0u : wid;
+    const uint32_t n0 = 32u * (W == 1u ? MM_WAVES * blockIdx.x + wid : blockIdx.x), m0 = 32u * blockIdx.y;
+    if (W == 1u && n0 >= N) return;
     const int8_t* bp = B + (size_t)min(n0 + r, N - 1u) * K;
     const int8_t* ap = A + (size_t)min(m0 + r, M - 1u) * lda;
     pf_i16 acc = {};
     const uint32_t full = K >> 5;
-    for (uint32_t s0 = wid; s0 < full; s0 += U * W) {
+    for (uint32_t s0 = part; s0 < full; s0 += U * W) {
         pf_i4 a[U], b[U];
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {   // past the last step: reloaded, not used
@@ -738,22 +754,35 @@ __global__ __launch_bounds__(64 * MM_WAVES) void k_matmul_i8(const int8_t* __res
         for (uint32_t u = 0; u < U; u++)
             if (s0 + u * W < full) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u], b[u], acc, 0, 0, 0);
     }
-    if ((K & 31u) && wid == full % W) {
+    if ((K & 31u) && part == full % W) {
         const uint32_t k = 32u * full + 16u * h;
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(row_tail16(ap, k, K), row_tail16(bp, k, K), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(tail16(A, (size_t)M * lda, (size_t)(ap - A), k, K),
+                                                    tail16(B, (size_t)N * K, (size_t)(bp - B), k, K), acc, 0, 0, 0);
     }
-#pragma unroll
-    for (uint32_t j = 0; j < 16; j++) red[wid][j][lane] = acc[j];
-    __syncthreads();
-    for (uint32_t x = t; x < 1024u; x += 64u * W) {
-        const uint32_t l = x & 63u, j = x >> 6;
-        const uint32_t m = m0 + 8u * (j >> 2) + 4u * (l >> 5) + (j & 3u), n = n0 + (l & 31u);
-        if (m >= M || n >= N) continue;
-        int v = red[0][j][l];
-#pragma unroll
-        for (uint32_t w = 1; w < W; w++) v += red[w][j][l];
+    auto put = [&](uint32_t m, uint32_t n, int v) {
         if constexpr (QUANT) C[(size_t)m * N + n] = (float)v * as[m] * ws[n];
         else Ci[(size_t)m * N + n] = v;
+    };
+    // sum j of lane (r, h): row 8 (j / 4) + 4 h + j % 4, column r of the tile
+    if constexpr (W == 1u) {
+#pragma unroll
+        for (uint32_t j = 0; j < 16; j++) {
+            const uint32_t m = m0 + 8u * (j >> 2) + 4u * h + (j & 3u), n = n0 + r;
+            if (m < M && n < N) put(m, n, acc[j]);
+        }
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < 16; j++) red[wid][j][lane] = acc[j];
+        __syncthreads();
+        for (uint32_t x = t; x < 1024u; x += 64u * W) {
+            const uint32_t l = x & 63u, j = x >> 6;
+            const uint32_t m = m0 + 8u * (j >> 2) + 4u * (l >> 5) + (j & 3u), n = n0 + (l & 31u);
+            if (m >= M || n >= N) continue;
+            int v = red[0][j][l];
+#pragma unroll
+            for (uint32_t w = 1; w < W; w++) v += red[w][j][l];
+            put(m, n, v);
+        }
     }
 }
 

@@ -778,8 +778,13 @@ extern "C" pf_status pf_quantize_activation_rows(pf_ctx* c, const float* src, in
 template <bool QUANT>
 static void launch_matmul_i8(hipStream_t st, const int8_t* A, uint32_t lda, const int8_t* B, uint32_t M, uint32_t N,
                              uint32_t K, int32_t* Ci, const float* as, const float* ws, float* C) {
-    hipLaunchKernelGGL(k_matmul_i8<QUANT>, dim3((N + 31) / 32, (M + 31) / 32), dim3(64 * MM_WAVES), 0, st, A, lda, B, M,
-                       N, K, Ci, as, ws, C);
+    const uint32_t nt = (N + 31) / 32, mt = (M + 31) / 32;
+    if (K <= MM_SHORT_K && (uint64_t)nt * mt >= MM_SHORT_TILES)
+        hipLaunchKernelGGL((k_matmul_i8<QUANT, 1>), dim3((nt + MM_WAVES - 1) / MM_WAVES, mt), dim3(64 * MM_WAVES), 0, st,
+                           A, lda, B, M, N, K, Ci, as, ws, C);
+    else
+        hipLaunchKernelGGL((k_matmul_i8<QUANT, MM_WAVES>), dim3(nt, mt), dim3(64 * MM_WAVES), 0, st, A, lda, B, M, N, K,
+                           Ci, as, ws, C);
 }
 
 extern "C" pf_status pf_matmul_int8(pf_ctx* c, const int8_t* A, const int8_t* B, int32_t* C, uint32_t M, uint32_t N,

@@ -41,10 +41,13 @@ def test_quantize_activation_rows(gpu):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (3, 33, 15), (1, 40, 16), (2, 31, 31), (33, 32, 33), (5, 77, 0),
-                                   (64, 65, 255), (31, 1000, 1100), (129, 4100, 47), (300, 4097, 130)])
+                                   (64, 65, 255), (31, 1000, 1100), (129, 4100, 47), (300, 4097, 130), (1, 3, 5),
+                                   (2, 3, 8), (40, 70, 4), (33, 65, 12), (5, 129, 17), (65, 33, 28),
+                                   (520, 4100, 100), (4100, 520, 5)])
 def test_matmul_i8_ragged(gpu, M, N, K):
-    """The MFMA int8 matmul at tile, step and row-tail edges and in each of
-    its tile shapes: integer sums equal, the scaled outputs bit for bit."""
+    """The MFMA int8 matmul at tile, step and row-tail edges (matrices of fewer
+    than 16 bytes among them), K over a workgroup's waves and a tile per wave:
+    integer sums equal, the scaled outputs bit for bit."""
     rng = np.random.default_rng(M * 1000 + K)
     A = rng.integers(-128, 128, (M, K), dtype=np.int8)
     B = rng.integers(-128, 128, (N, K), dtype=np.int8)
