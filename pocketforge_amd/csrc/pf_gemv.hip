@@ -711,7 +711,7 @@ __device__ __forceinline__ pf_i4 tail16(const int8_t* p, size_t total, size_t ro
 // of K with its operands straight from memory (16 bytes per lane, four steps'
 // loads together), and their int32 sums meet in LDS (exact, so the split
 // changes nothing).  QUANT: the outputs leave as (float)sum * as[i] * ws[j]
-// (src/matmul_neon.cpp:176-180), else as int32.
+// (src/matmul_neon.cpp:176-180), else as int32.  Columns from n_base on.
 //
 // Latency bounds the API's sizes (a few MB): splitting K over the waves puts
 // most of a workgroup's loads into one round trip.  M 100, N 3000, K 1100:
@@ -730,13 +730,13 @@ __global__ __launch_bounds__(64 * MM_WAVES) void k_matmul_i8(const int8_t* __res
                                                       const int8_t* __restrict__ B, uint32_t M, uint32_t N,
                                                       uint32_t K, int32_t* __restrict__ Ci,
                                                       const float* __restrict__ as, const float* __restrict__ ws,
-                                                      float* __restrict__ C) {
+                                                      float* __restrict__ C, uint32_t n_base) {
     static_assert(W == 1 || W == MM_WAVES, "a tile per wave or per workgroup");
     __shared__ int red[W][16][64];
     constexpr uint32_t U = 4;
     const uint32_t t = threadIdx.x, lane = t & 63u, r = lane & 31u, h = lane >> 5;
     const uint32_t wid = __builtin_amdgcn_readfirstlane(t >> 6), part = W == 1u ? 0u : wid;
-    const uint32_t n0 = 32u * (W == 1u ? MM_WAVES * blockIdx.x + wid : blockIdx.x), m0 = 32u * blockIdx.y;
+    const uint32_t n0 = n_base + 32u * (W == 1u ? MM_WAVES * blockIdx.x + wid : blockIdx.x), m0 = 32u * blockIdx.y;
     if (W == 1u && n0 >= N) return;
     const int8_t* bp = B + (size_t)min(n0 + r, N - 1u) * K;
     const int8_t* ap = A + (size_t)min(m0 + r, M - 1u) * lda;

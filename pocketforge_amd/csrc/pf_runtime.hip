@@ -775,22 +775,29 @@ extern "C" pf_status pf_quantize_activation_rows(pf_ctx* c, const float* src, in
     return PF_OK;
 }
 
+// A grid holds at most 2^32 - 1 threads per dimension: matrices of more than
+// MM_MAX_N columns take several launches.
+constexpr uint32_t MM_MAX_N = 1u << 27, MM_LAST_N = 0xFFFFFF00u;   // column indices of the last tiles fit 32 bits
 template <bool QUANT>
 static void launch_matmul_i8(hipStream_t st, const int8_t* A, uint32_t lda, const int8_t* B, uint32_t M, uint32_t N,
                              uint32_t K, int32_t* Ci, const float* as, const float* ws, float* C) {
-    const uint32_t nt = (N + 31) / 32, mt = (M + 31) / 32;
-    if (K <= MM_SHORT_K && (uint64_t)nt * mt >= MM_SHORT_TILES)
-        hipLaunchKernelGGL((k_matmul_i8<QUANT, 1>), dim3((nt + MM_WAVES - 1) / MM_WAVES, mt), dim3(64 * MM_WAVES), 0, st,
-                           A, lda, B, M, N, K, Ci, as, ws, C);
-    else
-        hipLaunchKernelGGL((k_matmul_i8<QUANT, MM_WAVES>), dim3(nt, mt), dim3(64 * MM_WAVES), 0, st, A, lda, B, M, N, K,
-                           Ci, as, ws, C);
+    const uint32_t mt = (M + 31) / 32;
+    for (uint64_t b = 0; b < N; b += MM_MAX_N) {
+        const uint32_t nb = (uint32_t)b, nt = (std::min(N - nb, MM_MAX_N) + 31) / 32;
+        if (K <= MM_SHORT_K && (uint64_t)nt * mt >= MM_SHORT_TILES)
+            hipLaunchKernelGGL((k_matmul_i8<QUANT, 1>), dim3((nt + MM_WAVES - 1) / MM_WAVES, mt), dim3(64 * MM_WAVES), 0,
+                               st, A, lda, B, M, N, K, Ci, as, ws, C, nb);
+        else
+            hipLaunchKernelGGL((k_matmul_i8<QUANT, MM_WAVES>), dim3(nt, mt), dim3(64 * MM_WAVES), 0, st, A, lda, B, M, N,
+                               K, Ci, as, ws, C, nb);
+    }
 }
 
 extern "C" pf_status pf_matmul_int8(pf_ctx* c, const int8_t* A, const int8_t* B, int32_t* C, uint32_t M, uint32_t N,
                                     uint32_t K) {
     if (!c || !A || !B || !C) return PF_ERR_ARG;
     if (M == 0 || N == 0) return PF_OK;
+    if (N > MM_LAST_N) return fail(c, PF_ERR_UNSUPPORTED, "N > 2^32 - 256");
     launch_matmul_i8<false>(c->stream, A, K, B, M, N, K, C, nullptr, nullptr, nullptr);
     PF_LAUNCHED(c);
     return PF_OK;
@@ -800,6 +807,7 @@ extern "C" pf_status pf_matmul_quantized(pf_ctx* c, const float* A, const int8_t
                                          uint32_t N, uint32_t K, const float* ws, const float* as_in) {
     if (!c || !A || !B || !C || !ws) return PF_ERR_ARG;
     if (M == 0 || N == 0) return PF_OK;
+    if (N > MM_LAST_N) return fail(c, PF_ERR_UNSUPPORTED, "N > 2^32 - 256");
     const uint32_t ldq = (K + 15u) / 16u * 16u;   // quantized rows start on 16 bytes
     const size_t q_bytes = ((size_t)M * ldq + 255) & ~(size_t)255;
     void* s = nullptr;

@@ -69,6 +69,19 @@ def test_matmul_i8_ragged(gpu, M, N, K):
         np.testing.assert_array_equal(got, ref)
 
 
+def test_matmul_int8_beyond_one_launch(gpu):
+    """More columns than one grid's threads cover (a tile per wave needs 2
+    threads per column, K over the waves 16)."""
+    N = (1 << 28) + 70
+    B = np.resize(np.arange(-128, 123, dtype=np.int8), N)
+    b, a, c = (pf.DeviceArray.from_numpy(gpu, x) for x in (B, np.array([3], np.int8), np.zeros(N, np.int32)))
+    gpu.check(pf.lib().pf_matmul_int8(gpu.h, a.ptr, b.ptr, c.ptr, 1, N, 1), "pf_matmul_int8")
+    gpu.synchronize()
+    assert (c.numpy() == np.multiply(B, 3, dtype=np.int32)).all()
+    for x in (a, b, c):
+        x.free()
+
+
 def test_matmul_int8_and_quantized(gpu):
     rng = np.random.default_rng(1)
     M, N, K = 5, 77, 300
