@@ -803,15 +803,24 @@ extern "C" pf_status pf_matmul_int8(pf_ctx* c, const int8_t* A, const int8_t* B,
     return PF_OK;
 }
 
+static bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + nb && y < x + na;
+}
+
 extern "C" pf_status pf_matmul_quantized(pf_ctx* c, const float* A, const int8_t* B, float* C, uint32_t M,
                                          uint32_t N, uint32_t K, const float* ws, const float* as_in) {
     if (!c || !A || !B || !C || !ws) return PF_ERR_ARG;
     if (M == 0 || N == 0) return PF_OK;
     if (N > MM_LAST_N) return fail(c, PF_ERR_UNSUPPORTED, "N > 2^32 - 256");
     const uint32_t ldq = (K + 15u) / 16u * 16u;   // quantized rows start on 16 bytes
-    const size_t q_bytes = ((size_t)M * ldq + 255) & ~(size_t)255;
+    const size_t q_bytes = ((size_t)M * ldq + 255) & ~(size_t)255, s_bytes = ((size_t)M * 4 + 255) & ~(size_t)255;
+    const size_t c_bytes = (size_t)M * N * 4;
+    // outputs over B or the given scales, which other workgroups still read,
+    // are formed apart and copied (A is quantized before)
+    const bool apart = overlap(C, c_bytes, B, (size_t)N * K) || (as_in && overlap(C, c_bytes, as_in, (size_t)M * 4));
     void* s = nullptr;
-    pf_status st = ctx_scratch(c, q_bytes + (size_t)M * 4, &s);
+    pf_status st = ctx_scratch(c, q_bytes + s_bytes + (apart ? c_bytes : 0), &s);
     if (st) return st;
     int8_t* Aq = (int8_t*)s;
     float* as = (float*)((char*)s + q_bytes);
@@ -822,8 +831,10 @@ extern "C" pf_status pf_matmul_quantized(pf_ctx* c, const float* A, const int8_t
         PF_PER_SWITCH(K, hipLaunchKernelGGL(k_quant_rows<PER>, dim3(M), dim3(256), 0, c->stream, A, K, K, Aq, ldq,
                                             as, (int32_t*)nullptr, 0u));
     }
-    launch_matmul_i8<true>(c->stream, Aq, ldq, B, M, N, K, nullptr, as_in ? as_in : as, ws, C);
+    float* out = apart ? (float*)((char*)as + s_bytes) : C;
+    launch_matmul_i8<true>(c->stream, Aq, ldq, B, M, N, K, nullptr, as_in ? as_in : as, ws, out);
     PF_LAUNCHED(c);
+    if (apart) PF_HIP(c, hipMemcpyAsync(C, out, c_bytes, hipMemcpyDeviceToDevice, c->stream));
     return PF_OK;
 }
 

@@ -82,6 +82,30 @@ def test_matmul_int8_beyond_one_launch(gpu):
         x.free()
 
 
+@pytest.mark.parametrize("where", ["B", "act_scales", "A"])
+def test_matmul_quantized_over_its_inputs(gpu, where):
+    """Outputs that take the place of an input the call still reads."""
+    M, N, K = 200, 1000, 300
+    rng = np.random.default_rng(4)
+    A = (rng.standard_normal((M, K)) * 0.5).astype(np.float32)
+    B = rng.integers(-127, 128, (N, K), dtype=np.int8)
+    ws = (rng.random(N) * 0.02 + 0.001).astype(np.float32)
+    act = (np.abs(A).max(1) / 120.0).astype(np.float32)
+    ref = np.zeros((M, N), np.float32)
+    O.lib().orc_matmul_quantized(O.ptr(A, O.f32p), O.ptr(B, O.i8p), O.ptr(ref, O.f32p), M, N, K, O.ptr(ws, O.f32p),
+                                 O.ptr(act, O.f32p))
+    a, b, w, s = _t(A), _t(B), _t(ws), _t(act)
+    host = np.zeros(M * N, np.float32)
+    src = {"B": B, "act_scales": act, "A": A}[where].reshape(-1).view(np.uint8)
+    host.view(np.uint8)[: src.size] = src
+    C = pf.DeviceArray.from_numpy(gpu, host)
+    ptr = {"A": a.ptr, "B": b.ptr, "act_scales": s.ptr, where: C.ptr}
+    gpu.check(pf.lib().pf_matmul_quantized(gpu.h, ptr["A"], ptr["B"], C.ptr, M, N, K, w.ptr, ptr["act_scales"]),
+              "pf_matmul_quantized")
+    gpu.synchronize()
+    np.testing.assert_array_equal(C.numpy().reshape(M, N), ref)
+
+
 def test_matmul_int8_and_quantized(gpu):
     rng = np.random.default_rng(1)
     M, N, K = 5, 77, 300
