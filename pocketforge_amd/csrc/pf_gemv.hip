@@ -334,6 +334,9 @@ __global__ __launch_bounds__(256, KS == 1 || GLU ? 2 : 3) void k_mm_f32(
                     }
                 } else {
                     q4_weights(q == 0 ? cw[0].x : (q == 1 ? cw[0].y : (q == 2 ? cw[0].z : cw[0].w)), d, nd, w);
+                    // two wait states between a VALU write and the MFMA that
+                    // reads it, which the compiler does not count for asm
+                    asm("s_nop 1" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]), "+v"(w[7]));
                 }
                 const float e[8] = {x.x, x.y, x.z, x.w, z.x, z.y, z.z, z.w};
 #pragma unroll
