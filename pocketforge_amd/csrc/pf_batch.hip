@@ -25,7 +25,7 @@ extern "C" uint32_t pf_batch_position(const pf_engine* e, uint32_t seq) {
 }
 
 // Prompt passes of one sequence: consecutive positions in passes of up to
-// one window (at most 512 rows), exactly as pf_generate's prefill.
+// one window, exactly as pf_generate's prefill.
 static pf_status batch_prefill_seq(pf_engine* e, uint32_t seq, const int32_t* tokens, uint32_t n) {
     pf_ctx* c = e->c;
     hipStream_t st = c->stream;
@@ -82,29 +82,36 @@ extern "C" pf_status pf_batch_forward(pf_engine* e, const uint32_t* seqs, uint32
         seen[seqs[i]] = 1;
     }
     batch_sync_in(e);
-    uint32_t pos_last = 0;
-    PassDesc& pd = e->pd_host;
-    pd.pos0 = 0;
-    pd.m = rows;
-    pd.batch = 1;
-    pd.seq0 = 0;
-    for (uint32_t i = 0; i < n; i++)
-        for (uint32_t j = 0; j < rows_per_seq; j++) {
-            const uint32_t r = i * rows_per_seq + j;
-            pd.tok[r] = tokens[r];
-            pd.rpos[r] = e->spos[seqs[i]] + j;
-            pd.rseq[r] = seqs[i];
-            pos_last = std::max(pos_last, pd.rpos[r]);
-        }
-    if ((uint64_t)pos_last + 1 > e->rope_pos) return fail(c, PF_ERR_CAPACITY, "position beyond the engine's max_context");
-    PF_HIP(c, hipMemcpyAsync(e->pdP, &pd, sizeof(PassDesc), hipMemcpyHostToDevice, c->stream));
-    PF_HIP(c, hipStreamSynchronize(c->stream));
-    pd.batch = 0;
-    e->batch_group = rows_per_seq;           // each sequence's rows_per_seq consecutive positions
-    pf_status s = run_pass(e, e->pdP, rows, 0, logits ? e->logitsB : nullptr, hidden ? e->hiddenB : nullptr, true,
-                           pos_last);
-    e->batch_group = 0;
-    if (s) return s;
+    uint32_t pos_hi = 0;
+    for (uint32_t i = 0; i < n; i++) pos_hi = std::max(pos_hi, e->spos[seqs[i]]);
+    if ((uint64_t)pos_hi + rows_per_seq > e->rope_pos)
+        return fail(c, PF_ERR_CAPACITY, "position beyond the engine's max_context");
+    // more rows of a sequence than the ring's slack (then it is the only one,
+    // 2 x 257 rows being more than a pass has) take several passes
+    const uint32_t step = std::min(rows_per_seq, MAX_PREFILL_ROWS);
+    for (uint32_t j0 = 0; j0 < rows_per_seq; j0 += step) {
+        const uint32_t nj = std::min(step, rows_per_seq - j0);
+        PassDesc& pd = e->pd_host;
+        pd.pos0 = 0;
+        pd.m = n * nj;
+        pd.batch = 1;
+        pd.seq0 = 0;
+        for (uint32_t i = 0; i < n; i++)
+            for (uint32_t j = 0; j < nj; j++) {
+                const uint32_t r = i * nj + j;
+                pd.tok[r] = tokens[i * rows_per_seq + j0 + j];
+                pd.rpos[r] = e->spos[seqs[i]] + j0 + j;
+                pd.rseq[r] = seqs[i];
+            }
+        PF_HIP(c, hipMemcpyAsync(e->pdP, &pd, sizeof(PassDesc), hipMemcpyHostToDevice, c->stream));
+        PF_HIP(c, hipStreamSynchronize(c->stream));
+        pd.batch = 0;
+        e->batch_group = nj;                 // each sequence's nj consecutive positions
+        pf_status s = run_pass(e, e->pdP, n * nj, 0, logits ? e->logitsB + (size_t)j0 * d.n_vocab : nullptr,
+                               hidden ? e->hiddenB + (size_t)j0 * d.n_embd : nullptr, true, pos_hi + j0 + nj - 1);
+        e->batch_group = 0;
+        if (s) return s;
+    }
     for (uint32_t i = 0; i < n; i++) e->spos[seqs[i]] += rows_per_seq;
     batch_sync_out(e);
     if (logits)

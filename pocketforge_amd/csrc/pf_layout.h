@@ -42,16 +42,15 @@ __host__ __device__ constexpr int code_offset(int fmt) {
 // One (layer, head) plane holds KV_SINK_ROWS sink rows, then `ring` window
 // slots (window index w lives in slot w % ring), then `pool_cap` pooled
 // rows.  K and V are separate planes of int8 [rows][head_dim] with fp32 row
-// scales [rows].  ring = window + pool_block + (rows of the tallest pass)
+// scales [rows].  ring = window + pool_block + (rows of the tallest pass that
+// evicts)
 // keeps every window entry alive until it has been folded into its pooled
 // row and lets a pass write its pending rows without touching visible
 // entries.
 constexpr uint32_t KV_SINK_ROWS = 8;
 constexpr uint32_t MAX_PASS_ROWS = 8;        // decode passes (verify: n_mtp + 1 rows)
-// Prompt passes (MFMA GEMMs and attention): 512 rows against 256 take 110
-// against 144 us per 512 rows in a 1B layer's products, and half the launches.
-constexpr uint32_t MAX_PREFILL_ROWS = 512;
-constexpr uint32_t MAX_FORWARD_ROWS = 256;   // rows of one pf_forward call without outputs
+// Rows of a prompt pass (MFMA GEMMs) wherever it lies, and the ring's slack.
+constexpr uint32_t MAX_PREFILL_ROWS = 256;
 constexpr uint32_t MAX_SEQS = 128;           // sequences of a multi-sequence engine
 constexpr uint32_t MAX_ROWS = 512;           // rows of any pass (batched verify: rows x sequences)
 

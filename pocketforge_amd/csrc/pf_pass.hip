@@ -316,6 +316,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                                                                                    dn.x, dn.nw);
 }
 
+// The descriptors of the groups of `group` rows of a pass of M consecutive
+// positions: all that the attention of a group reads.
+__global__ __launch_bounds__(64) void k_group_descs(const PassDesc* __restrict__ pd, uint32_t M, uint32_t group,
+                                                    PassDesc* __restrict__ sub) {
+    const uint32_t i = threadIdx.x;
+    if (i * group >= M) return;
+    sub[i].pos0 = pd->pos0 + i * group;
+    sub[i].m = min(group, M - i * group);
+    sub[i].batch = 0u;
+    sub[i].seq0 = pd->seq0;
+}
+
 // A pass's first launch: the pooled rows it can see (k_pool_rows, blocks
 // [0, n_pool): layers * heads per pooled-row slot ny) and its embedded rows
 // with the epoch advance (k_embed, 128 columns per block), two independent

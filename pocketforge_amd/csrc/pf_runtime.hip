@@ -633,15 +633,19 @@ static int per_for(uint32_t K) {
 // rows inside the attention kernel (FUSED); taller passes have them stored by
 // k_kv_store_pass first.
 static bool attn_fused(uint32_t M) { return M <= AG_MAX_ROWS; }
+// Whether prefix lists take k_attn_tile: its time is one workgroup's (22 us at
+// head_dim 128, 15 at 64) up to 256 workgroups, then 10 us per 256 more;
+// k_attn_group's grows with its blocks of 4 rows: 11.5 / 21 / 29 / 114 us at 192
+// / 384 / 576 / 2560 of them (head_dim 128), 9 / 16 us at 16 / 192 (head_dim 64)
+static bool attn_tiled(uint32_t hd, uint32_t M, uint32_t tasks) {
+    return M > AG_MAX_ROWS && (M + 3) / 4 * tasks > (hd == 64 ? 192u : 384u);
+}
+
 static void launch_attn(hipStream_t st, uint32_t hd, uint32_t M, uint32_t tasks, const PassDesc* pd,
                         const KvGeom& g, const KvPlanes& kv, uint32_t l, const float* q, const float* k,
                         const float* v, float* S, uint32_t s_stride, float* Wp, uint32_t cstride, Prefetch pf,
                         bool batch, uint32_t gsize, bool prefix, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr) {
-    // k_attn_tile's time is one workgroup's (22 us at head_dim 128, 15 at 64)
-    // up to 256 workgroups, then 10 us per 256 more; k_attn_group's grows with
-    // its blocks of 4 rows: 11.5 / 21 / 29 / 114 us at 192 / 384 / 576 / 2560 of
-    // them (head_dim 128), 9 / 16 us at 16 / 192 (head_dim 64)
-    if (prefix && !ev0 && M > AG_MAX_ROWS && (M + 3) / 4 * tasks > (hd == 64 ? 192u : 384u)) {
+    if (prefix && !ev0 && attn_tiled(hd, M, tasks)) {
         // blocks b with equal b mod 8 (one XCD) hold whole (head, chunk)
         // groups of 32-row tiles
         const uint32_t tiles = (M + 31) / 32;
@@ -1372,7 +1376,29 @@ static bool model_complete(const pf_model* m) {
 
 struct TimedPass { hipEvent_t a, b; bool verify; };
 
-struct pf_engine {
+// Where a pass's rows lie in the engine's pass memory.
+struct PassBufs {
+    float* x = nullptr;         // residual stream [rows][D]
+    int8_t* act = nullptr;      // quantized activation rows [rows][kmax]
+    float* as = nullptr;        // their row scales [4][as_rows]
+    uint32_t as_rows = 0;
+    float *q = nullptr, *k = nullptr, *v = nullptr;   // [rows][D] after RoPE
+    float* sg = nullptr;        // SwiGLU output [rows][F]
+    float* S = nullptr;         // attention chunks' maxima and sums, of `group` rows
+    float* Wp = nullptr;        // and weighted values
+    uint32_t s_stride = 0, cstride = 0;
+    uint32_t group = MAX_ROWS;  // rows whose attention runs together
+    PassDesc* sub = nullptr;    // descriptors of a pass's groups, where it has several
+};
+
+// The next n elements at offset `at` of mem, on a 256-byte boundary.
+template <class T>
+static void lay(T*& p, uint8_t* mem, size_t& at, size_t n) {
+    p = mem ? reinterpret_cast<T*>(mem + at) : nullptr;
+    at += (n * sizeof(T) + 255) & ~(size_t)255;
+}
+
+struct pf_engine : PassBufs {   // (the base: `rows` rows of every buffer)
     pf_model* m = nullptr;
     pf_ctx* c = nullptr;
     KvGeom g{};
@@ -1381,18 +1407,12 @@ struct pf_engine {
     float* rope_c = nullptr;
     float* rope_s = nullptr;
     uint32_t rope_pos = 0;
-    // pass scratch
-    float* x = nullptr;         // residual stream [rows][D]
-    int8_t* act = nullptr;      // quantized activation rows [rows][kmax]
-    float* as = nullptr;        // their row scales [4][rows]
-    float *q = nullptr, *k = nullptr, *v = nullptr;   // [rows][D] after RoPE
-    float* sg = nullptr;        // SwiGLU output [rows][F]
-    float* pmax = nullptr;      // its per-workgroup row maxima [8][2F / 32] (decode passes)
-    float* S = nullptr;
-    float* Wp = nullptr;
-    uint32_t s_stride = 0, cstride = 0, kmax = 0;
+    uint8_t* pass_mem = nullptr;
+    size_t pass_bytes = 0;
+    float* pmax = nullptr;      // per-workgroup row maxima of sg [8][2F / 32] (decode passes)
+    uint32_t kmax = 0;
     uint32_t cmax = 0;            // longest attention list (sink + pool + window)
-    uint32_t prefill_rows = 8;    // rows of a prompt pass
+    uint32_t prefill_rows = 8;    // rows of a pf_forward pass (prompt_rows: those of a prompt's)
     PassDesc pd_host{};           // staging of the prompt passes' descriptors
     float *logitsA = nullptr, *hiddenA = nullptr, *logitsB = nullptr, *hiddenB = nullptr;
     float *mcur = nullptr, *ma = nullptr, *mlogits = nullptr;
@@ -1576,9 +1596,7 @@ static pf_status engine_create(pf_model* m, const pf_cache_desc* cd, uint32_t ns
         PF_HIP(c, hipMemcpy(e->rope_s, sn.data(), sn.size() * 4, hipMemcpyHostToDevice));
     }
     e->kmax = std::max(D, F);
-    // prompt passes: at most one window of rows, so that every pooled row a
-    // pass sees was folded from entries stored before the pass
-    e->prefill_rows = std::min(PR, e->g.window);
+    e->prefill_rows = std::min(MAX_PREFILL_ROWS, e->g.window);
     const uint32_t cmax = KV_SINK_ROWS + e->g.pool_cap + e->g.window;
     if (H > 128 || (uint64_t)H * ((cmax + 1 + 255) / 256) > 2048) {
         pf_engine_destroy(e);
@@ -1590,15 +1608,20 @@ static pf_status engine_create(pf_model* m, const pf_cache_desc* cd, uint32_t ns
     if (const char* v = std::getenv("PF_PREFETCH_BLOCKS")) e->pf_blocks = (uint32_t)std::strtoul(v, nullptr, 10);
     if (const char* v = std::getenv("PF_L2_BLOCKS")) e->l2_blocks = 8u * ((uint32_t)std::strtoul(v, nullptr, 10) / 8u);
     if (!s) s = ealloc(e, &e->sink, 1);
-    if (!s) s = ealloc(e, &e->x, (size_t)PR * D);
-    if (!s) s = ealloc(e, &e->act, (size_t)PR * e->kmax);
-    if (!s) s = ealloc(e, &e->as, 4 * PR);
-    if (!s) s = ealloc(e, &e->q, (size_t)PR * D);
-    if (!s) s = ealloc(e, &e->k, (size_t)PR * D);
-    if (!s) s = ealloc(e, &e->v, (size_t)PR * D);
-    if (!s) s = ealloc(e, &e->S, (size_t)PR * H * e->s_stride);
-    if (!s) s = ealloc(e, &e->Wp, (size_t)PR * H * e->cstride * hd);
-    if (!s) s = ealloc(e, &e->sg, (size_t)PR * F);
+    e->as_rows = PR;
+    for (int place = 0; place < 2 && !s; place++) {   // sizes, then addresses
+        size_t at = 0;
+        lay(e->x, e->pass_mem, at, (size_t)PR * D);
+        lay(e->act, e->pass_mem, at, (size_t)PR * e->kmax);
+        lay(e->as, e->pass_mem, at, 4 * PR);
+        lay(e->q, e->pass_mem, at, (size_t)PR * D);
+        lay(e->k, e->pass_mem, at, (size_t)PR * D);
+        lay(e->v, e->pass_mem, at, (size_t)PR * D);
+        lay(e->S, e->pass_mem, at, (size_t)PR * H * e->s_stride);
+        lay(e->Wp, e->pass_mem, at, (size_t)PR * H * e->cstride * hd);
+        lay(e->sg, e->pass_mem, at, (size_t)PR * F);
+        if (!place) s = ealloc(e, &e->pass_mem, e->pass_bytes = at);
+    }
     if (!s) s = ealloc(e, &e->pmax, (size_t)GEMV_MAX_M * (2 * F / 32));
     if (!s) s = ealloc(e, &e->logitsA, (size_t)MA * V);
     if (!s) s = ealloc(e, &e->hiddenA, (size_t)MA * D);
@@ -2111,12 +2134,67 @@ static uint32_t prefix_end(const KvGeom& g) {
     return g.sink_size <= KV_SINK_ROWS ? std::min(g.max_context, g.sink_size + g.window) : 0u;
 }
 
-// Rows of the next prompt pass at position pos: one that starts before
-// prefix_end stops there, so that all of it can take the attention of prefix
-// lists.
+// The pass memory laid out for a prompt pass of more rows than the base
+// layout has: the SwiGLU rows take the place of the q/k/v rows (the attention
+// is done with them by then), and the chunk results are packed for the chunks
+// the pass sees and held for one group of rows at a time.  Returns the bytes.
+static size_t tall_layout(const pf_engine* e, uint32_t rows, uint32_t chunks, uint32_t group, uint8_t* mem, PassBufs* b) {
+    const size_t D = e->m->d.n_embd, F = e->m->d.n_ff, H = e->g.n_heads, hd = e->g.head_dim;
+    const size_t R = (rows + 31) / 32 * 32;
+    size_t at = 0;
+    b->as_rows = (uint32_t)R;
+    b->s_stride = 2 * chunks;
+    b->cstride = chunks;
+    b->group = group;
+    lay(b->x, mem, at, R * D);
+    lay(b->act, mem, at, R * e->kmax);
+    lay(b->as, mem, at, 4 * R);
+    lay(b->q, mem, at, R * std::max(3 * D, F));
+    if (mem) b->k = b->q + R * D, b->v = b->k + R * D;
+    b->sg = b->q;
+    lay(b->S, mem, at, group * H * b->s_stride);
+    lay(b->Wp, mem, at, group * H * b->cstride * hd);
+    lay(b->sub, mem, at, (rows + group - 1) / group);
+    return at;
+}
+
+static uint32_t list_chunks(const KvGeom& g, uint32_t pos) { return (kv_view(g, pos).count() + 1 + 255) / 256; }
+
+// Rows per attention group of a prompt pass of `rows` rows from pos (0: the
+// pass memory cannot hold it): all of them if they fit, but no more than the
+// ring's slack once the pass evicts, since a group's rows are stored together.
+static uint32_t tall_group(const pf_engine* e, uint32_t pos, uint32_t rows) {
+    const uint32_t last = pos + rows - 1, chunks = list_chunks(e->g, last);
+    uint32_t most = (rows + 31) / 32 * 32;
+    if (last > prefix_end(e->g)) most = std::min(most, MAX_PREFILL_ROWS);
+    PassBufs b;
+    for (uint32_t g = most; g; g -= 32)
+        if (tall_layout(e, rows, chunks, g, nullptr, &b) <= e->pass_bytes) {
+            const uint32_t n = (rows + g - 1) / g;
+            return ((rows + n - 1) / n + 31) / 32 * 32;   // groups of about one size
+        }
+    return 0;
+}
+
+// Rows of the next prompt pass at position pos: at most one window, so that
+// every pooled row the pass sees was folded from entries stored before it
+// (any number before prefix_end, where nothing is evicted), and as many as
+// the pass memory holds with at most two attention groups (layer skip stages
+// the base layout's rows).  512 rows against 256 take 110 against 144 us per
+// 512 rows in a 1B layer's products, and half the launches; a second group
+// costs a layer about 20 us.  A pass that would cross prefix_end stops there,
+// so that all of it can take the attention of prefix lists.
 static uint32_t prompt_rows(const pf_engine* e, uint32_t pos, uint32_t left) {
-    const uint32_t n = std::min(e->prefill_rows, left), end = prefix_end(e->g);
-    return pos < end && pos + n - 1 > end ? end + 1 - pos : n;
+    const uint32_t most = e->skip_on ? MAX_PREFILL_ROWS : MAX_ROWS, pr = std::min(most, e->g.window);
+    const uint32_t end = prefix_end(e->g), before = pos < end ? end + 1 - pos : 0u;
+    uint32_t n = std::min(pr, left);
+    if (before && n > before) {
+        n = before;
+    } else if (before && !e->skip_on) {
+        n = std::min({most, left, before});
+    }
+    while (n > MAX_PREFILL_ROWS && 2 * tall_group(e, pos, n) < n) n = (n - 1) / 32 * 32;
+    return n;
 }
 
 // One forward pass of M rows (the PassDesc at `pd` holds positions and
@@ -2131,8 +2209,8 @@ static uint32_t prompt_rows(const pf_engine* e, uint32_t pos, uint32_t left) {
 // prologue, SwiGLU epilogue), down product (quantize prologue, residual
 // epilogue): seven kernels.  Taller passes quantize their rows in row
 // kernels and run the GEMM with the same epilogues.
-static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0, float* logits, float* hidden,
-                          bool batch = false, uint32_t pos_last = 0) {
+static pf_status run_pass_rows(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0, float* logits, float* hidden,
+                               bool batch, uint32_t pos_last) {
     pf_ctx* c = e->c;
     const pf_model* m = e->m;
     const pf_model_desc& d = m->d;
@@ -2140,7 +2218,7 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
     hipStream_t st = c->stream;
     const uint32_t D = d.n_embd, F = d.n_ff, H = d.n_heads, hd = d.head_dim;
     if (!batch) pos_last = pos0 + M - 1;
-    if (M == 0 || M > e->rows) return fail(c, PF_ERR_ARG, "pass height beyond the engine's pass buffers");
+    if (M == 0 || M > e->as_rows) return fail(c, PF_ERR_ARG, "pass height beyond the engine's pass buffers");
     if (!e->capturing && pos_last + 1 > e->rope_pos)
         return fail(c, PF_ERR_CAPACITY, "position beyond the engine's max_context");
     // captured passes replay at any position: grids sized for the largest view
@@ -2152,11 +2230,13 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
     const bool merge_in_o = M == 1 && D <= 2048;
     // every row's list a prefix of the last row's (prefix_end)
     const bool prefix = !batch && !e->capturing && pos_last <= prefix_end(g);
-    // activation scales [4][rows] of the tall passes' row kernels
-    float* as0 = e->as;                   // attention-norm act
-    float* as1 = e->as + e->rows;         // attention output act
-    float* as2 = e->as + 2 * e->rows;     // ffn-norm act
-    float* as3 = e->as + 3 * e->rows;     // swiglu act
+    // activation scales [4][as_rows] of the tall passes' row kernels
+    float* as0 = e->as;                      // attention-norm act
+    float* as1 = e->as + e->as_rows;         // attention output act
+    float* as2 = e->as + 2 * e->as_rows;     // ffn-norm act
+    float* as3 = e->as + 3 * e->as_rows;     // swiglu act
+    if (M > e->group)
+        hipLaunchKernelGGL(k_group_descs, dim3(1), dim3(64), 0, st, (const PassDesc*)pd, M, e->group, e->sub);
 
     // pooled rows the pass can see (folded from window entries still in the ring)
     // and the embedded rows, in one launch (k_pass_prep)
@@ -2316,9 +2396,6 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
         }
         if (!qa)
             if (pf_status s = pass_mm(e, m->qkv[l], MM_QKV, M, a, as0)) return s;
-        if (!attn_fused(M))
-            hipLaunchKernelGGL(k_kv_store_pass, dim3(M, H), dim3(64), 0, st, (const PassDesc*)pd, g, e->kv, l,
-                               (const float*)e->k, (const float*)e->v);
         hipEvent_t aev0 = nullptr, aev1 = nullptr;
         if (e->profile == 1 && e->in_verify && !e->capturing) {
             if (e->aev_used == e->aev.size()) {
@@ -2362,16 +2439,32 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
             }
             if (hd == 64) qkv_attn_rows<4>(st, a, b, attn_tasks, aev0, aev1);
             else qkv_attn_rows<8>(st, a, b, attn_tasks, aev0, aev1);
-        } else {
-            launch_attn(st, hd, M, attn_tasks, pd, g, e->kv, l, e->q, e->k, e->v, e->S, e->s_stride, e->Wp,
-                        e->cstride, opf, batch, batch ? e->batch_group : 0u, prefix, aev0, aev1);
         }
-#define PF_MERGE(T)                                                                                                 \
-    PF_PER1024_SWITCH(D, hipLaunchKernelGGL((k_attn_merge_quant<PER, T>), dim3(M + e->pf_blocks), dim3(1024), 0, st, pd, \
-                                            g, (const float*)e->S, e->s_stride, (const float*)e->Wp, e->cstride,       \
-                                            e->act, ks, as1, (int32_t*)nullptr, 0u, M,                                 \
-                                            prefetch_of(e, m->o[l], e->pf_blocks)))
-        if (!merge_in_o && !tail) {
+#define PF_MERGE(T)                                                                                                    \
+    PF_PER1024_SWITCH(D, hipLaunchKernelGGL((k_attn_merge_quant<PER, T>), dim3(Mg + mpf.blocks), dim3(1024), 0, st, pg, g, \
+                                            (const float*)e->S, e->s_stride, (const float*)e->Wp, e->cstride,          \
+                                            e->act + o, ks, as1 + m0, (int32_t*)nullptr, 0u, Mg, mpf))
+        // the pass's rows, or a group of a prompt pass's after another; what a
+        // group that evicts stores may take the slot of an entry that the rows
+        // of the one before it still saw
+        const bool store_all = prefix && M > e->group;
+        if (store_all)
+            hipLaunchKernelGGL(k_kv_store_pass, dim3(M, H), dim3(64), 0, st, (const PassDesc*)pd, g, e->kv, l,
+                               (const float*)e->k, (const float*)e->v);
+        for (uint32_t m0 = 0; m0 < M && (!qa || !(merge_in_o || tail)); m0 += e->group) {
+            const uint32_t Mg = std::min(e->group, M - m0);
+            const PassDesc* pg = M > e->group ? e->sub + m0 / e->group : pd;
+            const size_t o = (size_t)m0 * D;
+            if (!store_all && !attn_fused(M))
+                hipLaunchKernelGGL(k_kv_store_pass, dim3(Mg, H), dim3(64), 0, st, pg, g, e->kv, l, (const float*)e->k + o,
+                                   (const float*)e->v + o);
+            const uint32_t tasks = M > e->group ? H * list_chunks(g, pos0 + m0 + Mg - 1) : attn_tasks;
+            if (!qa)
+                launch_attn(st, hd, Mg, tasks, pg, g, e->kv, l, e->q + o, e->k + o, e->v + o, e->S, e->s_stride, e->Wp,
+                            e->cstride, opf, batch, batch ? e->batch_group : 0u, prefix, aev0, aev1);
+            // the last group's merge also loads the O weights
+            const Prefetch mpf = prefetch_of(e, m->o[l], m0 + Mg == M ? e->pf_blocks : 0u);
+            if (merge_in_o || tail) continue;
             if (tall) {
                 PF_MERGE(true)
             } else {
@@ -2503,10 +2596,22 @@ static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0,
     return PF_OK;
 }
 
+static pf_status run_pass(pf_engine* e, PassDesc* pd, uint32_t M, uint32_t pos0, float* logits, float* hidden,
+                          bool batch = false, uint32_t pos_last = 0) {
+    if (batch || M <= MAX_PREFILL_ROWS) return run_pass_rows(e, pd, M, pos0, logits, hidden, batch, pos_last);
+    const uint32_t group = M <= MAX_ROWS ? tall_group(e, pos0, M) : 0u;
+    if (!group) return fail(e->c, PF_ERR_ARG, "pass height beyond the engine's pass buffers");
+    const PassBufs base = *e;
+    tall_layout(e, M, list_chunks(e->g, pos0 + M - 1), group, e->pass_mem, e);
+    const pf_status s = run_pass_rows(e, pd, M, pos0, logits, hidden, batch, pos_last);
+    static_cast<PassBufs&>(*e) = base;
+    return s;
+}
+
 extern "C" pf_status pf_forward(pf_engine* e, const int32_t* tokens, uint32_t n, float* logits, float* hidden) {
     if (!e || !tokens || n == 0) return PF_ERR_ARG;
     if (e->nseq != 1) return fail(e->c, PF_ERR_STATE, "multi-sequence engine: use pf_batch_forward");
-    if (n > ((logits || hidden) ? MAX_PASS_ROWS : std::min(MAX_FORWARD_ROWS, e->prefill_rows)))
+    if (n > ((logits || hidden) ? MAX_PASS_ROWS : e->prefill_rows))
         return fail(e->c, PF_ERR_ARG, "pass too tall: 8 rows with outputs, else one window up to 256 rows");
     if (e->pos + n > e->rope_pos) return fail(e->c, PF_ERR_CAPACITY, "position beyond the engine's max_context");
     pf_ctx* c = e->c;
@@ -2836,7 +2941,7 @@ extern "C" pf_status pf_generate(pf_engine* e, const int32_t* prompt, uint32_t n
     if (n_prompt) PF_HIP(c, hipMemcpyAsync(e->tokens, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice, st));
     auto t0 = std::chrono::steady_clock::now();
     // prefill (src/engine.cpp:286-290): every prompt token forwarded in order,
-    // in passes of up to one window (512 rows), whose GEMMs run on MFMA
+    // in passes of up to one window, whose GEMMs run on MFMA
     for (uint32_t i = 0, n; i < n_prompt; i += n) {
         n = prompt_rows(e, e->pos, n_prompt - i);
         e->pd_host.pos0 = e->pos;
