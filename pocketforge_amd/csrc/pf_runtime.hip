@@ -2182,14 +2182,20 @@ static uint32_t tall_group(const pf_engine* e, uint32_t pos, uint32_t rows) {
 // the pass memory holds with at most two attention groups (layer skip stages
 // the base layout's rows).  512 rows against 256 take 110 against 144 us per
 // 512 rows in a 1B layer's products, and half the launches; a second group
-// costs a layer about 20 us.  A pass that would cross prefix_end stops there,
-// so that all of it can take the attention of prefix lists.
+// costs a layer about 20 us.  A pass that would cross prefix_end stops there
+// if its rows up to there take the attention of prefix lists and the cut adds
+// no pass, or saves one's cost: TILE_CUT_BLOCKS blocks of 4 rows take 114 us
+// per layer, the same rows by tiles about 35, and a short pass's launches and
+// products about 60.
+constexpr uint32_t TILE_CUT_BLOCKS = 2560;
 static uint32_t prompt_rows(const pf_engine* e, uint32_t pos, uint32_t left) {
     const uint32_t most = e->skip_on ? MAX_PREFILL_ROWS : MAX_ROWS, pr = std::min(most, e->g.window);
     const uint32_t end = prefix_end(e->g), before = pos < end ? end + 1 - pos : 0u;
     uint32_t n = std::min(pr, left);
     if (before && n > before) {
-        n = before;
+        const uint32_t tasks = e->g.n_heads * list_chunks(e->g, end);
+        const bool free = (left - before + pr - 1) / pr <= (left - n + pr - 1) / pr;
+        if (attn_tiled(e->g.head_dim, before, tasks) && (free || (before + 3) / 4 * tasks > TILE_CUT_BLOCKS)) n = before;
     } else if (before && !e->skip_on) {
         n = std::min({most, left, before});
     }
