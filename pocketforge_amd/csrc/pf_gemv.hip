@@ -528,20 +528,20 @@ __global__ __launch_bounds__(256) void k_quant_rows(const float* __restrict__ x,
                                  bsum ? bsum + (size_t)m * bsum_stride : nullptr, red);
 }
 
-// quantize_activation_row of rows of length K <= 1024 * PER into the GEMM's
-// operand order, 1024 threads.
-template <int PER>
-__global__ __launch_bounds__(1024) void k_quant_rows_wide(const float* __restrict__ x, uint32_t K,
-                                                          int8_t* __restrict__ q, float* __restrict__ as) {
+// quantize_activation_row of rows of length K <= NT * PER into the GEMM's
+// operand order, NT threads.
+template <int PER, int NT = 1024>
+__global__ __launch_bounds__(NT) void k_quant_rows_wide(const float* __restrict__ x, uint32_t K,
+                                                        int8_t* __restrict__ q, float* __restrict__ as) {
     __shared__ float red[16];
     const uint32_t m = blockIdx.x;
     float v[PER];
 #pragma unroll
     for (int k = 0; k < PER; k++) {
-        const uint32_t i = threadIdx.x + 1024u * k;
+        const uint32_t i = threadIdx.x + (uint32_t)NT * k;
         v[k] = i < K ? x[(size_t)m * K + i] : 0.0f;
     }
-    quantize_row_block<PER, 1024, true>(v, K, q + operand_row(m, K), as + m, nullptr, red);
+    quantize_row_block<PER, NT, true>(v, K, q + operand_row(m, K), as + m, nullptr, red);
 }
 
 // LayerSkipController::should_skip_ffn (src/layer_skip.cpp:22-67) at one

@@ -437,10 +437,12 @@ static void gemm_split(hipStream_t st, const GemmArgs& a, hipEvent_t ev0, hipEve
 // once (two such workgroups per CU), else over four.  us with the row
 // quantization, 8 against 4 waves: 256 workgroups (256 rows of 2048 x 5632)
 // 18.7 / 22.8, 384 (128 rows of 6144 x 2048) 12.5 / 12.8, 704 (128 rows of
-// 11264 x 2048) 16.9 / 15.8, 1408 (256 rows) 27.1 / 25.2.
+// 11264 x 2048) 16.9 / 15.8, 1408 (256 rows) 27.1 / 25.2.  Below 1024 columns
+// (two steps a wave of eight) the waves' meeting costs more than the split
+// saves: 512 rows of 2048 x 256 took 9.1, with four waves 7.7.
 template <int F, int EPI, bool G>
 static void gemm_one(hipStream_t st, const GemmArgs& a, hipEvent_t ev0, hipEvent_t ev1) {
-    if ((a.M + 31) / 32 * (a.N / 64) <= 512) gemm_split<F, EPI, G, 8>(st, a, ev0, ev1);
+    if ((a.M + 31) / 32 * (a.N / 64) <= 512 && a.K >= 1024) gemm_split<F, EPI, G, 8>(st, a, ev0, ev1);
     else gemm_split<F, EPI, G, 4>(st, a, ev0, ev1);
 }
 
@@ -868,8 +870,12 @@ static pf_status gemv_q_run(pf_ctx* c, const pf_matrix* W, const float* x, float
         PF_LAUNCHED(c);
         return PF_OK;
     }
-    // 1024 threads a row: 5.0 us for 320 rows of 5632 where 256 threads take 9.0
-    PF_PER1024_SWITCH(K, hipLaunchKernelGGL(k_quant_rows_wide<PER>, dim3(M), dim3(1024), 0, c->stream, x, K, act, as));
+    // 1024 threads a row: 5.0 us for 320 rows of 5632 where 256 threads take 9.0;
+    // up to 1024 columns 256 (16 rows of 256 x 2048: 7.1 -> 6.1 us in all)
+    if (K <= 1024)
+        hipLaunchKernelGGL((k_quant_rows_wide<4, 256>), dim3(M), dim3(256), 0, c->stream, x, K, act, as);
+    else
+        PF_PER1024_SWITCH(K, hipLaunchKernelGGL(k_quant_rows_wide<PER>, dim3(M), dim3(1024), 0, c->stream, x, K, act, as));
     GemmArgs g{};
     g.W = W->data; g.N = N; g.K = K; g.M = M; g.act = act; g.as = as; g.e = e;
     launch_gemm(c->stream, W, MM_STORE, g);
