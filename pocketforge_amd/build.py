@@ -76,17 +76,22 @@ def build_forge():
 
 def build_cpp_tests():
     """The forge:: C++ tests, linked against libforge_amd.so and the oracle
-    (their checker).  Binaries go to _lib/tests/."""
+    (their checker), and the kernel tests (.hip, no library).  Binaries go to
+    _lib/tests/."""
     os.makedirs(TEST_BIN, exist_ok=True)
     out = []
     for f in sorted(os.listdir(CPP_TESTS)):
-        if not f.endswith(".cpp"):
+        src = os.path.join(CPP_TESTS, f)
+        exe = os.path.join(TEST_BIN, os.path.splitext(f)[0])
+        if f.endswith(".cpp"):
+            _run(["g++", "-O2", "-std=c++17", "-I" + os.path.join(ROOT, "include"), "-I" + CPP_TESTS,
+                  "-I" + os.path.join(ROOT, "oracle"), src, "-o", exe,
+                  "-L" + LIBDIR, "-lforge_amd", "-lpocketforge_amd", "-L" + ORACLE_BUILD, "-loracle",
+                  "-Wl,-rpath,$ORIGIN/..", "-Wl,-rpath,$ORIGIN/../../../oracle/_build"])
+        elif f.endswith(".hip"):
+            _run([HIPCC] + HIP_FLAGS + [src, "-o", exe])
+        else:
             continue
-        exe = os.path.join(TEST_BIN, f[:-4])
-        _run(["g++", "-O2", "-std=c++17", "-I" + os.path.join(ROOT, "include"), "-I" + CPP_TESTS,
-              "-I" + os.path.join(ROOT, "oracle"), os.path.join(CPP_TESTS, f), "-o", exe,
-              "-L" + LIBDIR, "-lforge_amd", "-lpocketforge_amd", "-L" + ORACLE_BUILD, "-loracle",
-              "-Wl,-rpath,$ORIGIN/..", "-Wl,-rpath,$ORIGIN/../../../oracle/_build"])
         out.append(exe)
     return out
 

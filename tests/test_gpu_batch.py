@@ -181,20 +181,43 @@ def test_unembedding_of_many_rows(gpu, n, d, vocab, fmt):
     m.close()
 
 
-@pytest.mark.parametrize("n_seq", [17, 28, 33])
+def _square_heads(w, d):
+    """Heads whose state is h + c relu(h)^2 (gate 16 x the identity, up and down
+    the identity, in 32-element blocks): the product decides the draft, so one of
+    another row, or with gate and up exchanged, is rejected."""
+    def diagonal(value):
+        codes = np.full((d, d // 32, 16), 0x88, np.uint8)
+        scales = np.zeros((d, d // 32), np.uint16)
+        for i in range(d):
+            codes[i, i // 32, i % 32 // 2] += 0x70 if i & 1 else 0x07
+            scales[i, i // 32] = np.float16(value / 7).view(np.uint16)
+        return (pf.FMT_Q4, codes, scales)
+    out = dict(w)
+    out["mtp"] = [dict(gate=diagonal(16384.0), up=diagonal(64.0), down=diagonal(64.0)) for _ in w["mtp"]]
+    return out
+
+
+@pytest.mark.parametrize("n_seq", [17, 18, 27, 28, 33, 64])
 def test_draft_heads_of_many_sequences(gpu, tiny_weights, n_seq):
     """The heads' gate|up and down products on either side of their
-    matrix-core thresholds: tokens equal a single engine's."""
+    matrix-core thresholds: tokens and accepted drafts equal a single engine's,
+    whose few-row products the oracle pins."""
     cfg, w = tiny_weights
-    m = pf.Model(gpu, cfg, _mix(w, 0.0005, 11))
+    m = pf.Model(gpu, cfg, _square_heads(_mix(w, 0.0005, 11), cfg["n_embd"]))
     b, e = pf.BatchEngine(m, n_seq, **KV), pf.Engine(m, **KV)
     prompts = [W.prompt_ids(5 + s % 7, cfg["n_vocab"], seed=s) for s in range(n_seq)]
-    toks, res = b.generate_batch(prompts, 12, TOP_P, np.arange(n_seq, dtype=np.uint64) + 3)
-    for s in (0, n_seq // 2, n_seq - 1):
+    toks, res = b.generate_batch(prompts, 12, GREEDY, np.arange(n_seq, dtype=np.uint64) + 3)
+    hidden = e.forward(prompts[0][:1])[1][0]
+    logits = e.mtp_forward(hidden)
+    assert not np.array_equal(logits[0], logits[1])     # a product of zeros would leave every head's logits the same
+    accepted = 0
+    for s in range(n_seq):
         e.reset()
-        t1, r1 = e.generate(prompts[s], 12, TOP_P, s + 3)
+        t1, r1 = e.generate(prompts[s], 12, GREEDY, s + 3)
         np.testing.assert_array_equal(toks[s], t1)
-        assert res[s].mtp_accepted == r1.mtp_accepted
+        assert (res[s].mtp_accepted, res[s].mtp_rejected) == (r1.mtp_accepted, r1.mtp_rejected)
+        accepted += r1.mtp_accepted
+    assert accepted >= 4 * n_seq
     b.close()
     e.close()
     m.close()

@@ -2,6 +2,9 @@
 import ctypes as C
 import os
 
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -449,3 +452,13 @@ def test_gemm_int8_block(gpu, fmt, shape):
             a8, s = O.quantize_activation_row(x[m])
             np.testing.assert_array_equal(y[m], O.gemv_i8(fmt, codes, scales, a8, s), err_msg=f"fmt {fmt} M {M} row {m}")
     W.close()
+
+
+def test_fp32_products_of_many_rows():
+    """k_mm_f32 with a head's gate and up in one launch, and with a residual,
+    against the few-row kernels bit for bit (tests/cpp/test_mm_f32.hip: no call
+    returns these products)."""
+    exe = os.path.join(os.path.dirname(pf.__file__), "_lib", "tests", "test_mm_f32")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    print(r.stdout, r.stderr, flush=True)
+    assert r.returncode == 0
