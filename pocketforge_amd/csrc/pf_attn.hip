@@ -1424,7 +1424,8 @@ __device__ __forceinline__ void attn_tile_v_rows(const pf_v32f& s, pf_v32f (&w)[
 // ns), so the two conversion steps per MFMA and the exps count in full: 256
 // MFMAs (8.4 us) and about 1500 VALU instructions (3.2 us) per wave at
 // head_dim 128.  In k_attn_group the VALU runs the chains and both conversions
-// for at most 4 rows per loaded chunk.  Three workgroups per CU (50 KB of LDS).
+// for at most 4 rows per loaded chunk.  Three workgroups per CU (50 KB of LDS),
+// whose 168 registers a lane spill two words at head_dim 128 (none at 64).
 // Measured per launch of 256 rows (16 heads of 128): 23.6 us at 2 chunks, 95
 // at 16, 134 at 23, 10 us per 256 workgroups once the chip is full; over a
 // 6000-token prompt 81 us on average, where k_attn_group took 490.

@@ -253,8 +253,8 @@ __global__ __launch_bounds__(256) void k_gemv_f32_glu(const uint8_t* __restrict_
 // matrix rows; one step of its loop forms blocks l and l + 32 (the
 // instruction's two halves) and adds them, the halving tree's first level.
 // Blocks come in bit-reversed order of l, so the deeper levels join as a
-// binary counter of partial tiles.  KS > 1 splits the blocks over KS waves of
-// the workgroup by the tree's last levels, whose partial tiles meet in LDS.
+// binary counter of partial tiles.  KS 4 splits the blocks over the workgroup's
+// waves by the tree's last two levels, whose partial tiles meet in LDS.
 // Blocks past K / 32 count as zeros, as k_gemv_f32's idle lanes do.
 //
 // Grid 8 * mtiles * ceil(n groups / 8), a group being the 4 / KS matrix tiles
@@ -274,7 +274,8 @@ __global__ __launch_bounds__(256, KS == 1 || GLU ? 2 : 3) void k_mm_f32(
     const float* __restrict__ y_in) {
     constexpr uint32_t NG = 4u / KS;                        // matrix tiles of a workgroup
     constexpr uint32_t CB = FMT == FMT_Q8 ? 2u : 1u;        // 16-byte code words per block
-    constexpr int LV = KS == 1 ? 5 : (KS == 2 ? 4 : 3);     // tree levels inside the wave
+    static_assert(KS == 1 || KS == 4, "a wave per tile, or the workgroup's four");
+    constexpr int LV = KS == 1 ? 5 : 3;                     // tree levels inside the wave
     __shared__ float red[KS > 1 ? 4 * 16 * 64 : 1];
     const uint32_t t = threadIdx.x, lane = t & 63u, r = lane & 31u, hh = lane >> 5;
     const uint32_t wid = __builtin_amdgcn_readfirstlane(t >> 6), part = wid % KS;
@@ -392,12 +393,9 @@ __global__ __launch_bounds__(256, KS == 1 || GLU ? 2 : 3) void k_mm_f32(
             __syncthreads();
             const uint32_t w0 = wid - part;
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                float x = red[(w0 * 16u + i) * 64u + lane] + red[((w0 + 1u) * 16u + i) * 64u + lane];
-                if constexpr (KS == 4)
-                    x = x + (red[((w0 + 2u) * 16u + i) * 64u + lane] + red[((w0 + 3u) * 16u + i) * 64u + lane]);
-                tot[i] = x;
-            }
+            for (int i = 0; i < 16; i++)
+                tot[i] = (red[(w0 * 16u + i) * 64u + lane] + red[((w0 + 1u) * 16u + i) * 64u + lane]) +
+                         (red[((w0 + 2u) * 16u + i) * 64u + lane] + red[((w0 + 3u) * 16u + i) * 64u + lane]);
         }
         if (GLU && prod == 0)
 #pragma unroll

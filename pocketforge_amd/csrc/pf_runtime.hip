@@ -577,7 +577,8 @@ static void launch_gemv_f32(hipStream_t st, const pf_matrix* W, uint32_t M, cons
 }
 
 // Gate and up products of one MTP head with the SiLU product fused:
-// a[m] = silu(Wg h[m]) * (Wu h[m]), rows in slices of F32_GROUP.
+// a[m] = silu(Wg h[m]) * (Wu h[m]), rows in slices of F32_GROUP; from GLU_TALL
+// rows on, the matrix core.
 static void launch_gemv_f32_glu(hipStream_t st, const pf_matrix* Wg, const pf_matrix* Wu, uint32_t M, const float* h,
                                 uint32_t h_stride, float* a, uint32_t a_stride, uint32_t max_waves = 2048) {
     if (M >= GLU_TALL) return mm_f32_one<FMT_Q4, true, 4>(st, Wg, Wu, M, h, h_stride, a, a_stride, nullptr);
